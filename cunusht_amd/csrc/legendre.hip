@@ -206,11 +206,6 @@ __global__ void k_prep(int lmax, int s, int nmaps, int nbpad, int ncomp, const d
 }
 
 // ------------------------------------------------------------------ synthesis kernel
-template <int NB>
-struct SynAcc0 {
-  double2 a[2][NB];
-};
-
 __device__ __forceinline__ void fma2(double2& acc, double2 c, double w) {
   acc.x = fma(c.x, w, acc.x);
   acc.y = fma(c.y, w, acc.y);
@@ -232,76 +227,91 @@ struct SynthArgs {
   long sm, sr, smap;
 };
 
-// One wave per (m, group of 64 ring pairs), starting at the group's first contributing l.
-// The l-loop runs in chunks of CH so that the wave-uniform coefficients of a chunk are fetched
-// together (one scalar-cache round trip per chunk instead of per l).  Tables are padded by CH
-// entries so a chunk never reads past the end.
-constexpr int kSynCH = 8;  // largest chunk of any variant (table padding)
+// Entries a chunked, prefetching l-loop may read past the last l of the last m: three chunks of 8 l (k_synth_row).
+constexpr int kSynPad = 32;
 
+// Every 8 l of the slow phase (some lane of the wave still below 2^-300): a chain whose scaled value passed 2^200
+// moves up one scale step.  A step of the recursion grows a value by at most sqrt(2 l + 3), so between two checks a
+// scaled value stays below 2^300, and what is masked until the next check is below 2^-300.
+constexpr double kRescale = 0x1p200;
+constexpr int kRescaleL = 8;
+static_assert(kStartAlign % kRescaleL == 0, "ring groups join the l-loop at a rescale check");
+
+__device__ __forceinline__ double rescaled_weight(double& mu, double& p, float& k) {
+  if (k < 0.f && fabs(mu) > kRescale) { mu *= kSmall; p *= kSmall; k += 1.f; }
+  return k == 0.f ? 1.0 : 0.0;
+}
+
+// One wave per (m, R groups of 64 ring pairs); each group joins the l-loop at its first contributing l.  The
+// coefficients are wave-uniform and arrive through the scalar cache in chunks of CH l, the next chunk's loads issued
+// before the current chunk's arithmetic (the tables are padded).  What bounds it: FP64 VALU issue.  Per l and ring pair
+// a spin-s E + B map takes 8 FMAs of contraction and 4 of recursion; the chip sustains one FP64 instruction per
+// 4.7 - 5.3 cycles and SIMD (clock and operand mix), and the loop runs at 5.6.  R: with one group per wave the
+// scalar-cache misses of the coefficient stream were the bound (loads from one fixed address: 8.0 -> 4.6 ms at lmax
+// 4095 spin 2), and R groups share one stream.  Measured at lmax 4095, one map, ms: spin 2 R = 1 / 2 / 3 / 4:
+// 7.1 / 6.07 / 6.7 / 8.1 (7.4 before, R = 1); spin-1 gradient 4.96 / 4.01 / 4.2 / 4.4 (4.66 before); spin 0 (chunks of
+// 4 l) R = 2 / 3 / 4: 3.2 / 2.84 / 2.76 (4.3 before, R = 1).  More groups lengthen the slow phase (4 % of the steps at
+// R = 1, 8 % at 2, 15 % at 4) and cost waves per SIMD.
 // GR (spin s, E only): the coefficient stream holds W' alone.  Since Wt' = (-1)^s conj(W') and the
 // recursion values are real, the -m sums are conjugates of the +m ones: the kernel accumulates
 // sum W' mu_u and sum W' mu_v split by the parity of l - l0 (half the contraction of the E + B case) and
 // forms the four ring coefficients at the end.
-template <bool SP, int NB, int CH, int WPB, bool GR = false>
-__global__ __launch_bounds__(64 * WPB) void k_synth(SynthArgs a) {
+template <bool SP, int NB, int R, int CH, bool GR, int MINW>
+__global__ __launch_bounds__(64, MINW) void k_synth(SynthArgs a) {
   static_assert(SP || !GR, "the gradient-only contraction is a spin-s case");
-  constexpr int R = 1;
+  static_assert(kRescaleL % CH == 0, "rescale checks fall on chunk starts");
   constexpr int K = (SP && !GR) ? 2 * NB : NB;
   // Blocks are dealt to the XCDs round-robin (block b runs on XCD b % 8).  XCD x takes
   // m = x, x + 8, x + 16, ... with all blocks of one m in a row, so each m's coefficient stream
-  // is read through one XCD's L2, and every XCD still starts with its longest m.  The WPB waves
-  // of a block take WPB adjacent slot groups of the same m and read the same coefficients, so
-  // all but the leading wave find them in the CU's scalar cache.
+  // is read through one XCD's L2, and every XCD still starts with its longest m.
   const int blk = blockIdx.x;
   const int j = blk / kNumXcd;
   const int m = (blk - j * kNumXcd) + kNumXcd * (j / a.nsb);
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int sb = (j % a.nsb) * WPB + wave;
+  const int sb = j % a.nsb;
   const int L = a.lmax;
   if (m > L) return;
   const int l0 = l0_of(m, a.s);
   // the launch may carry empty slot groups (odd block count per m, see launch_synth)
-  if (l0 > L || sb * 64 >= a.nslot) return;
-  const int lane = threadIdx.x & 63;
-  const int lstart = a.start[(long)m * ((a.nslot + 63) >> 6) + sb];
+  if (l0 > L || sb * 64 * R >= a.nslot) return;
+  const int lane = threadIdx.x;
+  const int ng = (a.nslot + 63) >> 6;
 
-  double x[R], mu_u[R], mu_v[R], pu[R], pv[R], ku[R], kv[R];
-  int slot[R];
+  double x[R], mu_u[R], mu_v[R], pu[R], pv[R];
+  float ku[R], kv[R];
+  int lst[R];  // first contributing l of each group (past lmax: never)
+  int lc = L + 1, lall = l0;
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    slot[r] = sb * 64 + lane;
-    x[r] = mu_u[r] = mu_v[r] = pu[r] = pv[r] = ku[r] = kv[r] = 0.0;
-    if (slot[r] < a.nslot) {
-      const long q = (long)m * a.sstride + slot[r];
-      x[r] = cos(a.slot_theta[slot[r]]);
-      const double2 sm = a.st_mu[q], sp = a.st_p[q], sk = a.st_k[q];
-      mu_u[r] = sm.x; pu[r] = sp.x; ku[r] = sk.x;
-      if (SP) { mu_v[r] = sm.y; pv[r] = sp.y; kv[r] = sk.y; }
-    }
+    const int g = sb * R + r;
+    const int slot = g * 64 + lane;
+    lst[r] = __builtin_amdgcn_readfirstlane(g < ng ? a.start[(long)m * ng + g] : L + 1);
+    lc = min(lc, lst[r]);
+    if (lst[r] <= L) lall = max(lall, lst[r]);
+    x[r] = slot < a.nslot ? cos(a.slot_theta[slot]) : 0.0;
+    mu_u[r] = mu_v[r] = pu[r] = pv[r] = 0.0;
+    ku[r] = kv[r] = 0.f;
   }
+  lc = __builtin_amdgcn_readfirstlane(lc);
+  lall = __builtin_amdgcn_readfirstlane(lall);
 
   const long base = a.mofs[m];
   const double2* __restrict__ rec = a.rec + base;
   const double2* __restrict__ cf = a.coef + base * K;
 
-  // spin 0: A0/A1 = parity-split sums; spin s: PN (+m north), MN (-m north), A (+m south), MS (-m south)
-  double2 A0[R][NB], A1[R][NB], PN[R][NB], MN[R][NB], MS0[R][NB], MS1[R][NB];
+  // spin 0: P / A even / odd sums.  Spin s: P (+m north), N (-m north), A (+m south), B (-m south), the south-ring
+  // sign alternation inside.  GR: sums of W' mu_u over even / odd l - l0 in P / N, of W' mu_v in A / B.
+  double2 P[R][NB], N[R][NB], A[R][NB], B[R][NB];
 #pragma unroll
   for (int r = 0; r < R; ++r)
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      A0[r][b] = A1[r][b] = PN[r][b] = MN[r][b] = MS0[r][b] = MS1[r][b] = double2{0.0, 0.0};
-    }
+    for (int b = 0; b < NB; ++b) P[r][b] = N[r][b] = A[r][b] = B[r][b] = double2{0.0, 0.0};
 
   struct Buf {
     double2 rc[CH];
     double2 cw[CH][K];
   };
-  // Wave-uniform coefficients of one chunk of CH consecutive l (scalar loads).  The loop below
-  // issues the loads of chunk c + 1 before it computes chunk c; the tables are padded by 2 CH
-  // entries for the prefetch past the last chunk.
-  auto load = [&](int lc, Buf& b) {
-    const int j0 = lc - l0;
+  auto load = [&](int l, Buf& b) {
+    const int j0 = l - l0;
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
       b.rc[i] = rec[j0 + i];
@@ -309,134 +319,302 @@ __global__ __launch_bounds__(64 * WPB) void k_synth(SynthArgs a) {
       for (int k = 0; k < K; ++k) b.cw[i][k] = cf[(long)(j0 + i) * K + k];
     }
   };
+  double fu[R], fv[R];  // 1, or 0 while the lane's chain is below range (slow phase)
+  // groups starting at l load their state; chains that left their scale step move up
+  auto join = [&](int l) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (l == lst[r]) {
+        const int slot = (sb * R + r) * 64 + lane;
+        if (slot < a.nslot) {
+          const long q = (long)m * a.sstride + slot;
+          const double2 sm = a.st_mu[q], sp = a.st_p[q], sk = a.st_k[q];
+          mu_u[r] = sm.x; pu[r] = sp.x; ku[r] = (float)sk.x;
+          if (SP) { mu_v[r] = sm.y; pv[r] = sp.y; kv[r] = (float)sk.y; }
+        }
+      }
+      fu[r] = rescaled_weight(mu_u[r], pu[r], ku[r]);
+      fv[r] = SP ? rescaled_weight(mu_v[r], pv[r], kv[r]) : 0.0;
+    }
+  };
   // One chunk (the first l at even l - l0).  SLOW: some lane may still be below the
-  // representable range (masked contributions, rescaling); FULL: all CH l <= L.
-  auto chunk = [&](int lc, const Buf& bf, auto slow_tag, auto full_tag) {
+  // representable range (masked contributions); FULL: all CH l <= L.
+  auto chunk = [&](int l, const Buf& bf, auto slow_tag, auto full_tag) {
     constexpr bool SLOW = decltype(slow_tag)::value;
     constexpr bool FULL = decltype(full_tag)::value;
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
-      if (!FULL && lc + i > L) break;
+      if (!FULL && l + i > L) break;
       const bool odd = (i & 1) != 0;
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         double wu = mu_u[r], wv = mu_v[r];
-        if (SLOW) { wu = ku[r] == 0.0 ? wu : 0.0; wv = kv[r] == 0.0 ? wv : 0.0; }
+        if (SLOW) { wu *= fu[r]; if (SP) wv *= fv[r]; }
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
           if (!SP) {
-            if (odd) fma2(A1[r][b], bf.cw[i][b], wu); else fma2(A0[r][b], bf.cw[i][b], wu);
+            if (odd) fma2(A[r][b], bf.cw[i][b], wu); else fma2(P[r][b], bf.cw[i][b], wu);
           } else if (GR) {
-            // MS0 / MS1 hold sum W' mu_u by parity here
             const double2 w = bf.cw[i][b];
-            if (odd) { fma2(MS1[r][b], w, wu); fma2(A1[r][b], w, wv); }
-            else { fma2(MS0[r][b], w, wu); fma2(A0[r][b], w, wv); }
+            if (odd) { fma2(N[r][b], w, wu); fma2(B[r][b], w, wv); }
+            else { fma2(P[r][b], w, wu); fma2(A[r][b], w, wv); }
           } else {
             const double2 w = bf.cw[i][2 * b], wt = bf.cw[i][2 * b + 1];
-            fma2(PN[r][b], w, wu);
-            fma2(MN[r][b], wt, wv);
-            if (odd) { fma2(A1[r][b], w, wv); fma2(MS1[r][b], wt, wu); }
-            else { fma2(A0[r][b], w, wv); fma2(MS0[r][b], wt, wu); }
+            fma2(P[r][b], w, wu);
+            fma2(N[r][b], wt, wv);
+            if (odd) { fma2(A[r][b], w, -wv); fma2(B[r][b], wt, -wu); }
+            else { fma2(A[r][b], w, wv); fma2(B[r][b], wt, wu); }
           }
         }
-      }
-      // the step past l = lmax reads a padded table entry; its result is never used
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
+        // the step past l = lmax reads a padded table entry; its result is never used
         const double t = bf.rc[i].x * x[r];
-        const double nu = fma(t + bf.rc[i].y, mu_u[r], -pu[r]);
+        const double nu = SP ? fma(t + bf.rc[i].y, mu_u[r], -pu[r]) : fma(t, mu_u[r], -pu[r]);
         pu[r] = mu_u[r]; mu_u[r] = nu;
         if (SP) {
           const double nv = fma(t - bf.rc[i].y, mu_v[r], -pv[r]);
           pv[r] = mu_v[r]; mu_v[r] = nv;
         }
-        if (SLOW) {
-          if (ku[r] < 0.0 && fabs(mu_u[r]) > kThresh) { mu_u[r] *= kSmall; pu[r] *= kSmall; ku[r] += 1.0; }
-          if (SP && kv[r] < 0.0 && fabs(mu_v[r]) > kThresh) { mu_v[r] *= kSmall; pv[r] *= kSmall; kv[r] += 1.0; }
-        }
       }
+      __builtin_amdgcn_sched_barrier(0);  // keeps the next l's products out of this one's registers
     }
   };
   auto any_under = [&]() {
     bool under = false;
 #pragma unroll
-    for (int r = 0; r < R; ++r) under |= (ku[r] < 0.0) || (kv[r] < 0.0);
+    for (int r = 0; r < R; ++r) under |= (ku[r] < 0.f) || (kv[r] < 0.f);
     return __any(under);
   };
   using T_ = std::true_type;
   using F_ = std::false_type;
-  int lc = lstart;
-  Buf cur, nxt;
-  load(lc, cur);
-  // slow phase: while some lane of the wave is still below 2^-300
-  while (lc <= L && any_under()) {
-    load(lc + CH, nxt);
-    if (lc + CH - 1 <= L) chunk(lc, cur, T_{}, T_{});
-    else chunk(lc, cur, T_{}, F_{});
-    cur = nxt;
-    lc += CH;
+  if (lc <= L) {
+    Buf cur, nxt;
+    load(lc, cur);
+    // slow phase: while a group has still to join or some lane is below 2^-300
+    while (lc <= L && (lc <= lall || any_under())) {
+      if (((lc - l0) & (kRescaleL - 1)) == 0) join(lc);
+      load(lc + CH, nxt);
+      if (lc + CH - 1 <= L) chunk(lc, cur, T_{}, T_{});
+      else chunk(lc, cur, T_{}, F_{});
+      cur = nxt;
+      lc += CH;
+    }
+    // fast phase, two chunks per iteration so that the two buffers alternate without copies
+    while (lc + 2 * CH - 1 <= L) {
+      load(lc + CH, nxt);
+      chunk(lc, cur, F_{}, T_{});
+      load(lc + 2 * CH, cur);
+      chunk(lc + CH, nxt, F_{}, T_{});
+      lc += 2 * CH;
+    }
+    if (lc + CH - 1 <= L) {
+      load(lc + CH, nxt);
+      chunk(lc, cur, F_{}, T_{});
+      cur = nxt;
+      lc += CH;
+    }
+    if (lc <= L) chunk(lc, cur, F_{}, F_{});
   }
-  // fast phase, two chunks per iteration so that the two buffers alternate without copies (the loads reach at
-  // most CH entries past lmax, as in the single-chunk step)
-  while (lc + 2 * CH - 1 <= L) {
-    load(lc + CH, nxt);
-    chunk(lc, cur, F_{}, T_{});
-    load(lc + 2 * CH, cur);
-    chunk(lc + CH, nxt, F_{}, T_{});
-    lc += 2 * CH;
-  }
-  if (lc + CH - 1 <= L) {
-    load(lc + CH, nxt);
-    chunk(lc, cur, F_{}, T_{});
-    cur = nxt;
-    lc += CH;
-  }
-  if (lc <= L) chunk(lc, cur, F_{}, F_{});
 
   const double sg0 = ((l0 + m) & 1) ? -1.0 : 1.0;  // (-1)^{l+m} for even (l - l0)
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    if (slot[r] >= a.nslot) continue;
-    const int rn = a.slot_north[slot[r]];
-    const int rs = a.slot_south[slot[r]];
+    const int slot = (sb * R + r) * 64 + lane;
+    if (slot >= a.nslot) continue;
+    const int rn = a.slot_north[slot];
+    const int rs = a.slot_south[slot];
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       if (b >= a.nmaps) break;
       double2* Gb = a.G + b * a.smap;
       if (!SP) {
-        double2 gn = cadd(A0[r][b], A1[r][b]);
-        double2 gs = double2{sg0 * (A0[r][b].x - A1[r][b].x), sg0 * (A0[r][b].y - A1[r][b].y)};
-        Gb[(long)m * a.sm + (long)rn * a.sr] = gn;
-        if (rs >= 0) Gb[(long)m * a.sm + (long)rs * a.sr] = gs;
-      } else if (GR) {
-        // north +m: sum W' mu_u; north -m: (-1)^s conj(sum W' mu_v); south +m: sg0 (A0 - A1);
-        // south -m: sg0 (-1)^s conj(even - odd of sum W' mu_u)
-        const double ss = (a.s & 1) ? -1.0 : 1.0;
-        const double2 pn = cadd(MS0[r][b], MS1[r][b]);
-        const double2 av = cadd(A0[r][b], A1[r][b]);
-        const double2 pS = double2{sg0 * (A0[r][b].x - A1[r][b].x), sg0 * (A0[r][b].y - A1[r][b].y)};
-        const double2 mN = double2{ss * av.x, -ss * av.y};
-        const double2 mS = double2{sg0 * ss * (MS0[r][b].x - MS1[r][b].x), -sg0 * ss * (MS0[r][b].y - MS1[r][b].y)};
+        Gb[(long)m * a.sm + (long)rn * a.sr] = cadd(P[r][b], A[r][b]);
+        if (rs >= 0) Gb[(long)m * a.sm + (long)rs * a.sr] = cscale(csub(P[r][b], A[r][b]), sg0);
+      } else {
+        double2 pN, mN, pS, mS;
+        if (GR) {
+          // north +m: sum W' mu_u; north -m: (-1)^s conj(sum W' mu_v); south +m: sg0 (even - odd of sum W' mu_v);
+          // south -m: sg0 (-1)^s conj(even - odd of sum W' mu_u)
+          const double ss = (a.s & 1) ? -1.0 : 1.0;
+          pN = cadd(P[r][b], N[r][b]);
+          mN = cscale(cconj(cadd(A[r][b], B[r][b])), ss);
+          pS = cscale(csub(A[r][b], B[r][b]), sg0);
+          mS = cscale(cconj(csub(P[r][b], N[r][b])), sg0 * ss);
+        } else {
+          pN = P[r][b];
+          mN = N[r][b];
+          pS = cscale(A[r][b], sg0);
+          mS = cscale(B[r][b], sg0);
+        }
         const long rowp = (long)(L + m) * a.sm, rowm = (long)(L - m) * a.sm;
-        Gb[rowp + (long)rn * a.sr] = pn;
+        Gb[rowp + (long)rn * a.sr] = pN;
         if (rs >= 0) Gb[rowp + (long)rs * a.sr] = pS;
         if (m > 0) {
           Gb[rowm + (long)rn * a.sr] = mN;
           if (rs >= 0) Gb[rowm + (long)rs * a.sr] = mS;
         }
-      } else {
-        double2 pS = double2{sg0 * (A0[r][b].x - A1[r][b].x), sg0 * (A0[r][b].y - A1[r][b].y)};
-        double2 mS = double2{sg0 * (MS0[r][b].x - MS1[r][b].x), sg0 * (MS0[r][b].y - MS1[r][b].y)};
-        const long rowp = (long)(L + m) * a.sm, rowm = (long)(L - m) * a.sm;
-        Gb[rowp + (long)rn * a.sr] = PN[r][b];
-        if (rs >= 0) Gb[rowp + (long)rs * a.sr] = pS;
-        if (m > 0) {
-          Gb[rowm + (long)rn * a.sr] = MN[r][b];
-          if (rs >= 0) Gb[rowm + (long)rs * a.sr] = mS;
-        }
       }
     }
   }
+}
+
+// ------------------------------------------------------------------ synthesis with few waves
+// Broadcast of lane I of each 16-lane row to the whole row.
+template <int I>
+__device__ __forceinline__ double row_bcast(double v) {
+  return __builtin_amdgcn_update_dpp(0.0, v, 0x150 + I, 0xF, 0xF, true);
+}
+
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<I + 1, N>(f);
+  }
+}
+
+// acc += (c of lanes I, I + 1 of the row) * w: the complex coefficient is the DPP operand of the two FMAs.  A DPP
+// read needs two wait states after a VALU write of its source (the buffers are copied in the slow phase).
+template <int I, bool NEG>
+__device__ __forceinline__ void row_fma2(double2& acc, double c, double w) {
+  if constexpr (NEG)
+    asm("s_nop 1\n\tv_fmac_f64_dpp %0, -%2, %3 row_newbcast:%4 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %1, -%2, %3 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+        : "+v"(acc.x), "+v"(acc.y) : "v"(c), "v"(w), "n"(I), "n"(I + 1));
+  else
+    asm("s_nop 1\n\tv_fmac_f64_dpp %0, %2, %3 row_newbcast:%4 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f64_dpp %1, %2, %3 row_newbcast:%5 row_mask:0xf bank_mask:0xf"
+        : "+v"(acc.x), "+v"(acc.y) : "v"(c), "v"(w), "n"(I), "n"(I + 1));
+}
+
+// One map, one wave per (m, group of 64 ring pairs) and, for spin s, chain (u: north +m and south -m; v: north -m and
+// south +m), for launches that leave SIMDs with one or two waves: there a wave issues one FP64 instruction per
+// 8 - 9 cycles and nothing hides a scalar load, which returns out of order, so every wait covers all of them.  The
+// coefficients come as vector loads instead, 16 doubles per register in each 16-lane row (8 l of the recursion
+// table, 4 or 8 of the map's), three chunks of 8 l deep, and reach the arithmetic as DPP row broadcasts; the two
+// chains run side by side in two waves.  Kernel time at lmax 255, ms (k_synth with R = 1 before): spin 2 0.036 -> 0.020,
+// spin-1 gradient 0.030 -> 0.020, spin 0 0.018 -> 0.013; at lmax 4095 it loses to k_synth (two broadcasts per l and
+// chain more).
+enum RowMode { kRowScalar, kRowGrad, kRowFull };
+
+template <int MODE>
+__global__ __launch_bounds__(64) void k_synth_row(SynthArgs a) {
+  constexpr bool SP = MODE != kRowScalar;
+  constexpr int NC = SP ? 2 : 1;              // chains
+  constexpr int CW = MODE == kRowFull ? 4 : 2;  // coefficient doubles per l
+  constexpr int CH = 8;
+  const int blk = blockIdx.x;
+  const int j = blk / kNumXcd;
+  const int m = (blk - j * kNumXcd) + kNumXcd * (j / (a.nsb * NC));
+  const int sc = j % (a.nsb * NC);
+  const int sb = sc / NC;
+  const bool vch = SP && (sc % NC);
+  const int L = a.lmax;
+  if (m > L) return;
+  const int l0 = l0_of(m, a.s);
+  if (l0 > L || sb * 64 >= a.nslot) return;
+  const int lane = threadIdx.x, row = lane & 15;
+  int lc = a.start[(long)m * ((a.nslot + 63) >> 6) + sb];
+  const int slot = sb * 64 + lane;
+  double x = 0.0, mu = 0.0, p = 0.0;
+  float kk = 0.f;
+  if (slot < a.nslot) {
+    const long q = (long)m * a.sstride + slot;
+    x = cos(a.slot_theta[slot]);
+    const double2 sm = a.st_mu[q], sp = a.st_p[q], sk = a.st_k[q];
+    mu = vch ? sm.y : sm.x;
+    p = vch ? sp.y : sp.x;
+    kk = (float)(vch ? sk.y : sk.x);
+  }
+  const long base = a.mofs[m];
+  const double* __restrict__ rec = reinterpret_cast<const double*>(a.rec + base) + row;
+  // the v chain takes (W~', W') where the u chain takes (W', W~')
+  const double* __restrict__ cf =
+      reinterpret_cast<const double*>(a.coef) + base * CW + (MODE == kRowFull && vch ? row ^ 2 : row);
+  const bool flip = vch && (row & 1);  // the v chain's -B_l
+  double2 P{0.0, 0.0}, Q{0.0, 0.0};    // full: north and (sign alternating) south sums; else even and odd sums
+  struct Buf {
+    double rc, cw[CW / 2];
+  };
+  auto load = [&](int l, Buf& b) {
+    const long j0 = l - l0;
+    b.rc = rec[2 * j0];
+#pragma unroll
+    for (int k = 0; k < CW / 2; ++k) b.cw[k] = cf[j0 * CW + 16 * k];
+  };
+  auto chunk = [&](int l, const Buf& bf, double f, auto slow_tag, auto full_tag) {
+    constexpr bool SLOW = decltype(slow_tag)::value;
+    constexpr bool FULL = decltype(full_tag)::value;
+    const double rc = flip ? -bf.rc : bf.rc;
+    static_for<0, CH>([&](auto ic) {
+      constexpr int i = decltype(ic)::value;
+      constexpr bool odd = (i & 1) != 0;
+      if (!FULL && l + i > L) return;
+      const double w = SLOW ? mu * f : mu;
+      if constexpr (MODE == kRowFull) {
+        row_fma2<(i & 3) * 4, false>(P, bf.cw[i >> 2], w);
+        row_fma2<(i & 3) * 4 + 2, odd>(Q, bf.cw[i >> 2], w);
+      } else {
+        row_fma2<2 * i, false>(odd ? Q : P, bf.cw[0], w);
+      }
+      const double t = SP ? fma(row_bcast<2 * i>(rc), x, row_bcast<2 * i + 1>(rc)) : row_bcast<2 * i>(rc) * x;
+      const double nu = fma(t, mu, -p);
+      p = mu;
+      mu = nu;
+    });
+    __builtin_amdgcn_sched_barrier(0);  // the next chunk's waits stay behind this chunk
+  };
+  using T_ = std::true_type;
+  using F_ = std::false_type;
+  if (lc <= L) {
+    Buf b0, b1, b2;
+    load(lc, b0);
+    load(lc + CH, b1);
+    while (lc <= L && __any(kk < 0.f)) {
+      const double f = rescaled_weight(mu, p, kk);
+      load(lc + 2 * CH, b2);
+      if (lc + CH - 1 <= L) chunk(lc, b0, f, T_{}, T_{});
+      else chunk(lc, b0, f, T_{}, F_{});
+      b0 = b1;
+      b1 = b2;
+      lc += CH;
+    }
+    while (lc + 3 * CH - 1 <= L) {
+      load(lc + 2 * CH, b2);
+      chunk(lc, b0, 1.0, F_{}, T_{});
+      load(lc + 3 * CH, b0);
+      chunk(lc + CH, b1, 1.0, F_{}, T_{});
+      load(lc + 4 * CH, b1);
+      chunk(lc + 2 * CH, b2, 1.0, F_{}, T_{});
+      lc += 3 * CH;
+    }
+    while (lc + CH - 1 <= L) {
+      load(lc + 2 * CH, b2);
+      chunk(lc, b0, 1.0, F_{}, T_{});
+      b0 = b1;
+      b1 = b2;
+      lc += CH;
+    }
+    if (lc <= L) chunk(lc, b0, 1.0, F_{}, F_{});
+  }
+  if (slot >= a.nslot) return;
+  const double sg0 = ((l0 + m) & 1) ? -1.0 : 1.0;
+  const int rn = a.slot_north[slot], rs = a.slot_south[slot];
+  double2 north, south;
+  if constexpr (MODE == kRowFull) {
+    north = P;
+    south = cscale(Q, sg0);
+  } else {
+    north = cadd(P, Q);
+    south = cscale(csub(P, Q), sg0);
+    if constexpr (MODE == kRowGrad) {  // the -m rows (north of the v chain, south of the u chain): (-1)^s conj
+      const double ss = (a.s & 1) ? -1.0 : 1.0;
+      if (vch) north = cscale(cconj(north), ss);
+      else south = cscale(cconj(south), ss);
+    }
+  }
+  const long rowp = (long)(SP ? L + m : m) * a.sm, rowm = (long)(L - m) * a.sm;
+  if (!vch || m > 0) a.G[(vch ? rowm : rowp) + (long)rn * a.sr] = north;
+  if (rs >= 0 && (!SP || vch || m > 0)) a.G[((SP && !vch) ? rowm : rowp) + (long)rs * a.sr] = south;
 }
 
 // ------------------------------------------------------------------ synthesis on the matrix cores
@@ -1127,9 +1305,9 @@ void LegendreTables::build(int L, int s, const std::vector<double>& theta, hipSt
     nblk += ceil_div((long)(mo[m + 1] - mo[m]), 4L);
   }
   upload(mblk, mb);
-  // padded so that a chunked, prefetching l-loop may read up to 2 kSynCH entries past the last one
-  rec.alloc(sizeof(double2) * (size_t)(std::max<long>(nlm, 1) + 2 * kSynCH));
-  cnorm.alloc(sizeof(double) * (size_t)(std::max<long>(nlm, 1) + 2 * kSynCH));
+  // padded so that a chunked, prefetching l-loop may read past the last l of the last m
+  rec.alloc(sizeof(double2) * (size_t)(std::max<long>(nlm, 1) + kSynPad));
+  cnorm.alloc(sizeof(double) * (size_t)(std::max<long>(nlm, 1) + kSynPad));
   sstride = nslot;
   ngroups = ceil_div(nslot, 64);
   const size_t nst = (size_t)(L + 1) * sstride;
@@ -1168,8 +1346,8 @@ void LegendreTables::build(int L, int s, const std::vector<double>& theta, hipSt
 static int padded_maps(int nmaps) { return nmaps <= 1 ? 1 : nmaps <= 2 ? 2 : nmaps <= 4 ? 4 : 8; }
 
 size_t legendre_coef_bytes(const LegendreTables& t, int nmaps) {
-  // padded by 2 kSynCH entries (chunked, prefetching reads past the last l of the last m)
-  const size_t vec = sizeof(double2) * (size_t)(std::max<long>(t.nlm, 1) + 2 * kSynCH) * padded_maps(nmaps) *
+  // padded by kSynPad entries (chunked, prefetching reads past the last l of the last m)
+  const size_t vec = sizeof(double2) * (size_t)(std::max<long>(t.nlm, 1) + kSynPad) * padded_maps(nmaps) *
                      (t.spin ? 2 : 1);
   if (nmaps < 3) return vec;
   // matrix-core layout: 32 doubles per chain, map group and block of 4 l, 2 blocks of padding (prefetch)
@@ -1178,29 +1356,36 @@ size_t legendre_coef_bytes(const LegendreTables& t, int nmaps) {
   return std::max(vec, mf);
 }
 
-// Synthesis variants (l-chunk CH, waves per block WPB); the autotuner picks one per table.
-struct SynVariant {
-  int CH, WPB;
-};
-static const SynVariant kSynVariants[] = {{2, 1}, {2, 4}, {4, 4}, {2, 8}};
-constexpr int kNumSynVariants = 4;
+// Synthesis variants of one map, in order of the launch size they suit: k_synth_row, k_synth with few and with more
+// ring groups per wave; the autotuner picks one per table.  Launches of two maps take one group per wave
+// (k_synth<.., 2, 1, 2, ..>: the second map's accumulators take the registers of a second group).
+static const char* const kSynVariants[] = {"row broadcasts", "few groups per wave", "more groups per wave"};
+constexpr int kNumSynVariants = 3;
 
 template <bool SP, int NB, bool GR = false>
 static void launch_synth(const SynthArgs& a, int variant, hipStream_t st) {
   // Odd number of blocks per m: blocks are handed to XCDs and shader engines round-robin, and
   // with a power-of-two count every engine would see the same slot groups for every m, so the
   // polar groups (long underflow phases) would pile up on a few engines.
-  const int wpb = kSynVariants[variant].WPB;
-  const int nsb = ceil_div(ceil_div(a.nslot, 64), wpb) | 1;
-  const int nblocks = nsb * ceil_div(a.lmax + 1, kNumXcd) * kNumXcd;
   SynthArgs b = a;
-  b.nsb = nsb;
-  const dim3 blk(64 * wpb);
-  switch (variant) {
-    case 0: hipLaunchKernelGGL((k_synth<SP, NB, 2, 1, GR>), dim3(nblocks), blk, 0, st, b); break;
-    case 1: hipLaunchKernelGGL((k_synth<SP, NB, 2, 4, GR>), dim3(nblocks), blk, 0, st, b); break;
-    case 2: hipLaunchKernelGGL((k_synth<SP, NB, 4, 4, GR>), dim3(nblocks), blk, 0, st, b); break;
-    default: hipLaunchKernelGGL((k_synth<SP, NB, 2, 8, GR>), dim3(nblocks), blk, 0, st, b); break;
+  const auto blocks = [&](int groups, int chains) {
+    b.nsb = ceil_div(a.nslot, 64 * groups) | 1;
+    return dim3((unsigned)(b.nsb * chains * ceil_div(a.lmax + 1, kNumXcd) * kNumXcd));
+  };
+  if constexpr (NB > 1) {
+    hipLaunchKernelGGL((k_synth<SP, NB, 1, 2, GR, 1>), blocks(1, 1), dim3(64), 0, st, b);
+  } else if (variant == 0) {
+    constexpr int MODE = !SP ? kRowScalar : GR ? kRowGrad : kRowFull;
+    const dim3 grid = blocks(1, SP ? 2 : 1);
+    hipLaunchKernelGGL(k_synth_row<MODE>, grid, dim3(64), 0, st, b);
+  } else if (SP) {
+    const dim3 grid = blocks(variant, 1);
+    if (variant == 1) hipLaunchKernelGGL((k_synth<SP, 1, 1, 2, GR, 8>), grid, dim3(64), 0, st, b);
+    else hipLaunchKernelGGL((k_synth<SP, 1, 2, 2, GR, 6>), grid, dim3(64), 0, st, b);
+  } else {
+    const dim3 grid = blocks(variant + 1, 1);
+    if (variant == 1) hipLaunchKernelGGL((k_synth<SP, 1, 2, 4, GR, 6>), grid, dim3(64), 0, st, b);
+    else hipLaunchKernelGGL((k_synth<SP, 1, 3, 4, GR, 4>), grid, dim3(64), 0, st, b);
   }
   NUSHT_LAUNCH_CHECK();
 }
@@ -1403,8 +1588,8 @@ void legendre_autotune(LegendreTables& t, int ncomp, double2* coef_ws, double2* 
     float ms = 0;
     NUSHT_HIP(hipEventElapsedTime(&ms, e0, e1));
     if (verbose)
-      fprintf(stderr, "[nusht] legendre autotune %s lmax %d spin %d pairs %d: variant %d (CH %d, %d waves) %.3f ms\n",
-              t.tag.c_str(), t.lmax, t.spin, t.nslot, v, kSynVariants[v].CH, kSynVariants[v].WPB, ms / 2);
+      fprintf(stderr, "[nusht] legendre autotune %s lmax %d spin %d ncomp %d pairs %d: variant %d (%s) %.3f ms\n",
+              t.tag.c_str(), t.lmax, t.spin, ncomp, t.nslot, v, kSynVariants[v], ms / 2);
     if (ms < best) { best = ms; bestv = v; }
   }
   slot = bestv;
