@@ -2,9 +2,10 @@
 //
 // Replaces the reference's SHTns synth / analys / synth_grad calls
 // (cunusht/sht/GPU_sht_transformer.py:56-96) with per-m three-term recursions:
-//   synthesis : one wave per (m, block of 64 ring pairs); coefficients are wave-uniform
-//               and arrive through the scalar cache; the l-loop runs in two phases, first
-//               with underflow rescaling while any lane is still below 2^-300, then plain.
+//   synthesis : one wave per (m, one to three groups of 64 ring pairs); coefficients are wave-uniform
+//               and arrive through the scalar cache (small transforms: as vector loads and DPP row
+//               broadcasts); the l-loop runs in two phases, first with underflow rescaling while any
+//               lane is still below 2^-300, then plain.
 //   adjoint   : one workgroup per m holding all ring pairs (4 per lane); per-l sums over
 //               lanes are formed with a butterfly transpose-reduce in registers, summed over
 //               waves with LDS atomics, then written once.
@@ -491,9 +492,10 @@ __device__ __forceinline__ void row_fma2(double2& acc, double c, double w) {
 // 8 - 9 cycles and nothing hides a scalar load, which returns out of order, so every wait covers all of them.  The
 // coefficients come as vector loads instead, 16 doubles per register in each 16-lane row (8 l of the recursion
 // table, 4 or 8 of the map's), three chunks of 8 l deep, and reach the arithmetic as DPP row broadcasts; the two
-// chains run side by side in two waves.  Kernel time at lmax 255, ms (k_synth with R = 1 before): spin 2 0.036 -> 0.020,
-// spin-1 gradient 0.030 -> 0.020, spin 0 0.018 -> 0.013; at lmax 4095 it loses to k_synth (two broadcasts per l and
-// chain more).
+// chains run side by side in two waves.  With the coefficient preparation, ms, against the faster of k_synth with few
+// and with more groups: lmax 255 spin 2 0.033 -> 0.015, spin-1 gradient 0.027 -> 0.017, spin 0 0.022 -> 0.013;
+// lmax 1000 0.218 -> 0.160, 0.182 -> 0.125, 0.118 -> 0.070.  From lmax 1500 on (spin s) k_synth is the faster one
+// (two broadcasts per l and chain less): lmax 4095 spin 2 6.9 here, 4.8 there.
 enum RowMode { kRowScalar, kRowGrad, kRowFull };
 
 template <int MODE>
