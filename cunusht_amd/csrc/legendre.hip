@@ -6,9 +6,8 @@
 //               and arrive through the scalar cache (small transforms: as vector loads and DPP row
 //               broadcasts); the l-loop runs in two phases, first with underflow rescaling while any
 //               lane is still below 2^-300, then plain.
-//   adjoint   : one workgroup per m holding all ring pairs (4 per lane); per-l sums over
-//               lanes are formed with a butterfly transpose-reduce in registers, summed over
-//               waves with LDS atomics, then written once.
+//   adjoint   : the same waves; per-l sums over the lanes are formed in registers (halving steps over
+//               lane swaps) and added to the output with atomics, a last pass scales them.
 #include "legendre.h"
 
 #include "timing.h"
@@ -22,6 +21,9 @@
 
 namespace nusht {
 namespace {
+
+// What a kernel transforms: a spin-0 field, the E component of a spin-s field alone, or E and B.
+enum FieldMode { kScalar, kGrad, kFull };
 
 __host__ __device__ inline int l0_of(int m, int s) { return m > s ? m : s; }
 
@@ -496,13 +498,11 @@ __device__ __forceinline__ void row_fma2(double2& acc, double c, double w) {
 // and with more groups: lmax 255 spin 2 0.033 -> 0.015, spin-1 gradient 0.027 -> 0.017, spin 0 0.022 -> 0.013;
 // lmax 1000 0.218 -> 0.160, 0.182 -> 0.125, 0.118 -> 0.070.  From lmax 1500 on (spin s) k_synth is the faster one
 // (two broadcasts per l and chain less): lmax 4095 spin 2 6.9 here, 4.8 there.
-enum RowMode { kRowScalar, kRowGrad, kRowFull };
-
 template <int MODE>
 __global__ __launch_bounds__(64) void k_synth_row(SynthArgs a) {
-  constexpr bool SP = MODE != kRowScalar;
+  constexpr bool SP = MODE != kScalar;
   constexpr int NC = SP ? 2 : 1;              // chains
-  constexpr int CW = MODE == kRowFull ? 4 : 2;  // coefficient doubles per l
+  constexpr int CW = MODE == kFull ? 4 : 2;  // coefficient doubles per l
   constexpr int CH = 8;
   const int blk = blockIdx.x;
   const int j = blk / kNumXcd;
@@ -531,7 +531,7 @@ __global__ __launch_bounds__(64) void k_synth_row(SynthArgs a) {
   const double* __restrict__ rec = reinterpret_cast<const double*>(a.rec + base) + row;
   // the v chain takes (W~', W') where the u chain takes (W', W~')
   const double* __restrict__ cf =
-      reinterpret_cast<const double*>(a.coef) + base * CW + (MODE == kRowFull && vch ? row ^ 2 : row);
+      reinterpret_cast<const double*>(a.coef) + base * CW + (MODE == kFull && vch ? row ^ 2 : row);
   const bool flip = vch && (row & 1);  // the v chain's -B_l
   double2 P{0.0, 0.0}, Q{0.0, 0.0};    // full: north and (sign alternating) south sums; else even and odd sums
   struct Buf {
@@ -552,7 +552,7 @@ __global__ __launch_bounds__(64) void k_synth_row(SynthArgs a) {
       constexpr bool odd = (i & 1) != 0;
       if (!FULL && l + i > L) return;
       const double w = SLOW ? mu * f : mu;
-      if constexpr (MODE == kRowFull) {
+      if constexpr (MODE == kFull) {
         row_fma2<(i & 3) * 4, false>(P, bf.cw[i >> 2], w);
         row_fma2<(i & 3) * 4 + 2, odd>(Q, bf.cw[i >> 2], w);
       } else {
@@ -602,13 +602,13 @@ __global__ __launch_bounds__(64) void k_synth_row(SynthArgs a) {
   const double sg0 = ((l0 + m) & 1) ? -1.0 : 1.0;
   const int rn = a.slot_north[slot], rs = a.slot_south[slot];
   double2 north, south;
-  if constexpr (MODE == kRowFull) {
+  if constexpr (MODE == kFull) {
     north = P;
     south = cscale(Q, sg0);
   } else {
     north = cadd(P, Q);
     south = cscale(csub(P, Q), sg0);
-    if constexpr (MODE == kRowGrad) {  // the -m rows (north of the v chain, south of the u chain): (-1)^s conj
+    if constexpr (MODE == kGrad) {  // the -m rows (north of the v chain, south of the u chain): (-1)^s conj
       const double ss = (a.s & 1) ? -1.0 : 1.0;
       if (vch) north = cscale(cconj(north), ss);
       else south = cscale(cconj(south), ss);
@@ -918,21 +918,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NS == 1 ? 3 
 }
 
 // ------------------------------------------------------------------ adjoint kernel
-template <bool SP> struct AdjCfg {
-  static constexpr int R = SP ? 3 : 4;          // ring pairs per lane per pass
-  static constexpr int MaxThreads = 768;
-};
-
-// Sum of K complex values per lane over the 64 lanes of a wave (butterfly transpose-reduce).
-// Each step exchanges half of the remaining values with lane ^ off and keeps the other half,
-// so after log2(K) steps every lane holds one fully lane-summed element; the remaining steps
-// are plain all-reduce butterflies.  Lane ln ends up with element reduce_index<K>(ln).
-// The exchanges are VALU lane moves, not LDS permutes: lane ^ 32 and lane ^ 16 by the gfx950 permlane
-// swaps (v_permlane32_swap: lanes 32..63 of the first operand with lanes 0..31 of the second;
-// v_permlane16_swap: the odd 16-lane rows of the first with the even rows of the second; with both operands
-// the value itself, the lane's partner value is in one of the two results), lane ^ 8 by a DPP rotation by 8
-// inside each 16-lane row.  The closing all-reduce over the lanes that hold one element (16 for K = 4, 8 for
-// K = 8) adds the row rotation by 8 (16 lanes only), the half-row mirror and the quad swaps 2 and 1.
+// Lane exchanges of the sums over a wave's 64 ring pairs.
 template <int CTRL>
 __device__ __forceinline__ double dpp_mov(double v) {
   int lo = __double2loint(v), hi = __double2hiint(v);
@@ -940,112 +926,61 @@ __device__ __forceinline__ double dpp_mov(double v) {
   hi = __builtin_amdgcn_mov_dpp(hi, CTRL, 0xF, 0xF, false);
   return __hiloint2double(hi, lo);
 }
-constexpr int kDppRowRor8 = 0x128, kDppRowHalfMirror = 0x141, kDppQuadXor2 = 0x4E, kDppQuadXor1 = 0xB1;
+constexpr int kDppQuadXor2 = 0x4E, kDppQuadXor1 = 0xB1, kDppQuadSame = 0xE4;
+constexpr int kDppRowRor8 = 0x128, kDppRowShl4 = 0x104, kDppRowShr4 = 0x114;
 
-// the value of lane ^ OFF
-template <int OFF>
-__device__ __forceinline__ double lane_xor(double v) {
-  if constexpr (OFF == 8) {
-    return dpp_mov<kDppRowRor8>(v);
-  } else {
-    static_assert(OFF == 16 || OFF == 32, "lane exchanges at offsets 32, 16 and 8");
-    const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
-    const bool first = ((threadIdx.x & 63) & OFF) == 0;
-    if constexpr (OFF == 32) {
-      const auto rl = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
-      const auto rh = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
-      return __hiloint2double((int)(first ? rh[1] : rh[0]), (int)(first ? rl[1] : rl[0]));
-    } else {
-      const auto rl = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
-      const auto rh = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
-      return __hiloint2double((int)(first ? rh[1] : rh[0]), (int)(first ? rl[1] : rl[0]));
-    }
-  }
-}
-
-// a + (a of lane ^ OFF) in the lanes with (lane & OFF) == 0, b + (b of lane ^ OFF) in the others, for OFF = 32
-// or 16: one swap of the register pair per half does it.  permlane32_swap(x, y) leaves x = (own x | y of lane
-// - 32) and y = (x of lane + 32 | own y) over the two halves, permlane16_swap the same over the row pairs, so
-// x + y is the wanted sum in every lane.
+// a + (a of lane ^ OFF) in the lanes with (lane & OFF) == 0, b + (b of lane ^ OFF) in the others.
+// OFF = 32 or 16: one swap of the register pair per half does it.  permlane32_swap(x, y) leaves x = (own x | y of
+// lane - 32) and y = (x of lane + 32 | own y) over the two halves, permlane16_swap the same over the row pairs, so
+// x + y is the wanted sum in every lane.  OFF = 8 or 4: DPP moves inside the 16-lane row, the bank mask (groups of 4
+// lanes) choosing whose value a lane takes.
 template <int OFF>
 __device__ __forceinline__ double pair_sum(double a, double b) {
-  const unsigned alo = (unsigned)__double2loint(a), ahi = (unsigned)__double2hiint(a);
-  const unsigned blo = (unsigned)__double2loint(b), bhi = (unsigned)__double2hiint(b);
-  static_assert(OFF == 16 || OFF == 32, "pair sums at offsets 32 and 16");
+  static_assert(OFF == 32 || OFF == 16 || OFF == 8 || OFF == 4, "lane exchanges at offsets 32, 16, 8 and 4");
+  const int alo = __double2loint(a), ahi = __double2hiint(a), blo = __double2loint(b), bhi = __double2hiint(b);
   if constexpr (OFF == 32) {
-    const auto rl = __builtin_amdgcn_permlane32_swap(alo, blo, false, false);
-    const auto rh = __builtin_amdgcn_permlane32_swap(ahi, bhi, false, false);
+    const auto rl = __builtin_amdgcn_permlane32_swap((unsigned)alo, (unsigned)blo, false, false);
+    const auto rh = __builtin_amdgcn_permlane32_swap((unsigned)ahi, (unsigned)bhi, false, false);
+    return __hiloint2double((int)rh[0], (int)rl[0]) + __hiloint2double((int)rh[1], (int)rl[1]);
+  } else if constexpr (OFF == 16) {
+    const auto rl = __builtin_amdgcn_permlane16_swap((unsigned)alo, (unsigned)blo, false, false);
+    const auto rh = __builtin_amdgcn_permlane16_swap((unsigned)ahi, (unsigned)bhi, false, false);
     return __hiloint2double((int)rh[0], (int)rl[0]) + __hiloint2double((int)rh[1], (int)rl[1]);
   } else {
-    const auto rl = __builtin_amdgcn_permlane16_swap(alo, blo, false, false);
-    const auto rh = __builtin_amdgcn_permlane16_swap(ahi, bhi, false, false);
-    return __hiloint2double((int)rh[0], (int)rl[0]) + __hiloint2double((int)rh[1], (int)rl[1]);
+    constexpr int kFromUp = OFF == 8 ? kDppRowRor8 : kDppRowShl4;    // the value of lane + OFF
+    constexpr int kFromDown = OFF == 8 ? kDppRowRor8 : kDppRowShr4;  // the value of lane - OFF
+    constexpr int kLow = OFF == 8 ? 0x3 : 0x5, kHigh = OFF == 8 ? 0xC : 0xA;
+    const auto partner = [&](int x, int y) {
+      const int t = __builtin_amdgcn_update_dpp(0, x, kFromUp, 0xF, kLow, false);
+      return __builtin_amdgcn_update_dpp(t, y, kFromDown, 0xF, kHigh, false);
+    };
+    const auto own = [&](int x, int y) { return __builtin_amdgcn_update_dpp(x, y, kDppQuadSame, 0xF, kHigh, false); };
+    return __hiloint2double(own(ahi, bhi), own(alo, blo)) + __hiloint2double(partner(ahi, bhi), partner(alo, blo));
   }
 }
 
-template <int K, int k, int off>
-__device__ __forceinline__ void tr_step(double2 (&v)[K], int ln) {
-  if constexpr (k > 1) {
-    constexpr int half = k / 2;
-    const bool h = (ln & off) != 0;
+// Sums of 16 values per lane over the wave: halving steps (each lane keeps half of the values, added to its
+// partner's) over lane bits 5 to 2, then plain sums over the quad; lane ln ends up with the sum of value ln >> 2.
+__device__ __forceinline__ double wave_sums(double (&v)[16]) {
 #pragma unroll
-    for (int i = 0; i < half; ++i) {
-      if constexpr (off >= 16) {
-        v[i] = double2{pair_sum<off>(v[i].x, v[i + half].x), pair_sum<off>(v[i].y, v[i + half].y)};
-      } else {
-        const double2 keep = h ? v[i + half] : v[i];
-        const double2 send = h ? v[i] : v[i + half];
-        v[i] = double2{keep.x + lane_xor<off>(send.x), keep.y + lane_xor<off>(send.y)};
-      }
-    }
-    tr_step<K, half, off / 2>(v, ln);
-  } else {
-    double x = v[0].x, y = v[0].y;
-    if constexpr (off == 8) {
-      x += dpp_mov<kDppRowRor8>(x);
-      y += dpp_mov<kDppRowRor8>(y);
-    }
-    x += dpp_mov<kDppRowHalfMirror>(x);
-    y += dpp_mov<kDppRowHalfMirror>(y);
-    x += dpp_mov<kDppQuadXor2>(x);
-    y += dpp_mov<kDppQuadXor2>(y);
-    x += dpp_mov<kDppQuadXor1>(x);
-    y += dpp_mov<kDppQuadXor1>(y);
-    v[0] = double2{x, y};
-  }
-}
-
-template <int K>
-__device__ __forceinline__ double2 transpose_reduce(double2 (&v)[K]) {
-  static_assert(K == 4 || K == 8, "the lane exchanges cover K = 4 and K = 8");
-  tr_step<K, K, 32>(v, (int)(threadIdx.x & 63));
-  return v[0];
-}
-
-template <int K>
-__device__ __forceinline__ int reduce_index() {
-  const int ln = threadIdx.x & 63;
-  int idx = 0, k = K, off = 32;
+  for (int i = 0; i < 8; ++i) v[i] = pair_sum<32>(v[i], v[i + 8]);
 #pragma unroll
-  for (int step = 0; step < 6; ++step) {
-    if (k > 1) {
-      int half = k / 2;
-      if (ln & off) idx += half;
-      k = half;
-    }
-    off >>= 1;
-  }
-  return idx;
+  for (int i = 0; i < 4; ++i) v[i] = pair_sum<16>(v[i], v[i + 4]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) v[i] = pair_sum<8>(v[i], v[i + 2]);
+  double r = pair_sum<4>(v[0], v[1]);
+  r += dpp_mov<kDppQuadXor2>(r);
+  r += dpp_mov<kDppQuadXor1>(r);
+  return r;
 }
 
 struct AdjArgs {
-  int lmax, s, nslot, sstride, ngroups, ncomp;
+  int lmax, s, nslot, sstride, ngroups, nsb;
   const double* slot_theta;
   const int* slot_north;
   const int* slot_south;
   const long* mofs;
   const double2* rec;
-  const double* cnorm;
   const double2* st_mu;
   const double2* st_p;
   const double2* st_k;
@@ -1055,196 +990,219 @@ struct AdjArgs {
   double2* alm;
 };
 
-template <bool SP>
-__global__ __launch_bounds__(AdjCfg<SP>::MaxThreads) void k_adjoint(AdjArgs a) {
-  constexpr int kAdjR = AdjCfg<SP>::R;
-  extern __shared__ double2 lacc[];
-  const int m = blockIdx.x;
+// One wave per (m, R groups of 64 ring pairs), as in the synthesis: every wave runs its own l-range, so polar groups,
+// which contribute late or never, hold nobody up.  (One workgroup per m with all its ring pairs and an LDS sum per l
+// filled a CU at lmax 4095 and waited for its equatorial waves.)  Per K l the wave adds up its ring pairs' products in
+// registers, sums them over its lanes (wave_sums) and adds the 16 totals to the output array with one atomic each
+// (128 bytes, or 64 bytes of E and of B): the array (cleared before) holds, per (l, m),
+//   spin 0: sum, E alone: (-1)^s X + Y, E + B: X in E's place and Y in B's,
+// X and Y the sums over the u and v halves; k_adjoint_finish turns them into alm.  The recursion table comes as
+// vector loads, 8 l per register and 16-lane row, two chunks ahead, broadcast by DPP.
+// What bounds it: FP64 VALU issue.  Per l and ring pair a spin-s E + B map takes 8 FMAs and 4 of recursion, and the
+// lane sums (12 permlane swap pairs, 21 DPP and 14 adds per 4 l, a swap taking two issue slots) cost 7.5 / R more.
+// Times, ms, with the clearing and finishing passes (0.16 at lmax 4095): spin 2 lmax 4095 R = 1 / 2 / 3 / 4:
+// 13.4 / 10.2 / 9.3 / 9.6 (13.9 before), spin 0 6.1 / 4.2 / 3.65 / 3.7 (10.1 before); lmax 300 spin 2 0.040 / 0.047 /
+// 0.053 (0.131 before): few waves want the shorter l-step.
+template <int MODE, int R>
+__global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
+  constexpr bool SP = MODE != kScalar;
+  constexpr int NA = MODE == kFull ? 4 : 2;  // doubles per (l, m)
+  constexpr int K = 16 / NA;                 // l per lane sum
+  constexpr int CH = 8;
+  const int blk = blockIdx.x;
+  const int j = blk / kNumXcd;
+  const int m = (blk - j * kNumXcd) + kNumXcd * (j / a.nsb);
+  const int sb = j % a.nsb;
   const int L = a.lmax;
+  if (m > L) return;
   const int l0 = l0_of(m, a.s);
-  const long nalm = (long)(L + 1) * (L + 2) / 2;
-  const long mbase = (long)m * (2 * L + 1 - m) / 2;
-  if (l0 > L) {
-    for (int l = m + threadIdx.x; l <= L; l += blockDim.x) {
-      for (int c = 0; c < a.ncomp; ++c) a.alm[c * nalm + mbase + l] = double2{0.0, 0.0};
-    }
-    return;
-  }
-  const int nl = L - l0 + 1;
-  constexpr int NA = SP ? 2 : 1;
-  for (int i = threadIdx.x; i < nl * NA; i += blockDim.x) lacc[i] = double2{0.0, 0.0};
-
-  __syncthreads();
+  if (l0 > L || sb * 64 * R >= a.nslot) return;
+  const int lane = threadIdx.x;
   const long base = a.mofs[m];
-  const double2* __restrict__ rec = a.rec + base;
-  const double sgA = ((l0 + m) & 1) ? -1.0 : 1.0;  // (-1)^{l+m} at l = l0
-  constexpr int K = SP ? 4 : 8;
-  const int ridx = reduce_index<K>();
-  const bool writer = ((threadIdx.x & 63) & (64 / K - 1)) == 0;
-  const int nthr = blockDim.x;
-  const int cap = nthr * kAdjR;
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int lane = threadIdx.x & 63;
+  const double* __restrict__ rec = reinterpret_cast<const double*>(a.rec + base) + (lane & 15);
 
-  for (int pass0 = 0; pass0 < a.nslot; pass0 += cap) {
-  // per-lane ring pairs: the wave takes kAdjR adjacent groups of 64 ring pairs; group r joins
-  // the l-loop at its first contributing l, lst[r]
-  double x[kAdjR], mu[kAdjR], pm[kAdjR], ku[kAdjR];
-  double nv_[kAdjR], pv[kAdjR], kv[kAdjR];
-  double2 P0[kAdjR], P1[kAdjR], Q0[kAdjR], Q1[kAdjR];  // spin 0: E/O in P0/P1; spin s: PN, PS, QN, QS
-  int lst[kAdjR];
-  int lmin = L + 1;
+  // C[r]: the ring pair's factors.  The south-ring sign (-1)^{l+m} is sgA at even l - l0 and -sgA at odd ones:
+  //   spin 0: C0 / C1 = north +- south (even / odd l - l0)
+  //   E + B:  X = sum C0 u +- C1 v, Y = sum C2 v +- C3 u
+  //   E:      Z = (-1)^s X + Y = sum (C0 or C1) u + (C2 or C3) v (even or odd l - l0)
+  double x[R], mu[R], pm[R], nv[R], pv[R];
+  float ku[R], kv[R];
+  double2 C0[R], C1[R], C2[R], C3[R];
+  int lst[R];
+  int lc = L + 1, lall = l0;
+  const double sgA = ((l0 + m) & 1) ? -1.0 : 1.0;
 #pragma unroll
-  for (int r = 0; r < kAdjR; ++r) {
-    const int g = (pass0 >> 6) + wave * kAdjR + r;
+  for (int r = 0; r < R; ++r) {
+    const int g = sb * R + r;
+    lst[r] = __builtin_amdgcn_readfirstlane(g < a.ngroups ? a.start[(long)m * a.ngroups + g] : L + 1);
+    lc = min(lc, lst[r]);
+    if (lst[r] <= L) lall = max(lall, lst[r]);
     const int slot = g * 64 + lane;
-    lst[r] = g < a.ngroups ? a.start[(long)m * a.ngroups + g] : L + 1;
-    lmin = min(lmin, lst[r]);
-    x[r] = mu[r] = pm[r] = ku[r] = nv_[r] = pv[r] = kv[r] = 0.0;
-    P0[r] = P1[r] = Q0[r] = Q1[r] = double2{0.0, 0.0};
-    if (slot < a.nslot) {
-      const long q = (long)m * a.sstride + slot;
+    x[r] = mu[r] = pm[r] = nv[r] = pv[r] = 0.0;
+    ku[r] = kv[r] = 0.f;
+    C0[r] = C1[r] = C2[r] = C3[r] = double2{0.0, 0.0};
+    if (slot < a.nslot && lst[r] <= L) {
       x[r] = cos(a.slot_theta[slot]);
-      const double2 sm = a.st_mu[q], sp = a.st_p[q], sk = a.st_k[q];
-      mu[r] = sm.x; pm[r] = sp.x; ku[r] = sk.x;
-      if (SP) { nv_[r] = sm.y; pv[r] = sp.y; kv[r] = sk.y; }
       const int rn = a.slot_north[slot];
-      int rs = a.slot_south[slot];
-      if (rs == rn) rs = -1;
-      // the south-ring sign (-1)^{l+m} is sgA at even chunk positions and -sgA at odd ones (chunks start at
-      // l0 plus multiples of 4): sgA is folded in here, the alternation into the l-loop's unrolled FMAs
-      if (!SP) {
-        double2 gn = a.G[(long)m * a.sm + (long)rn * a.sr];
-        double2 gs = rs >= 0 ? a.G[(long)m * a.sm + (long)rs * a.sr] : double2{0.0, 0.0};
-        P0[r] = sgA > 0 ? cadd(gn, gs) : csub(gn, gs);  // taken at even positions
-        P1[r] = sgA > 0 ? csub(gn, gs) : cadd(gn, gs);  // taken at odd positions
+      const int rs = a.slot_south[slot];
+      const double2 zero{0.0, 0.0};
+      if constexpr (!SP) {
+        const double2* g0 = a.G + (long)m * a.sm;
+        const double2 gn = g0[(long)rn * a.sr];
+        const double2 gs = rs >= 0 ? cscale(g0[(long)rs * a.sr], sgA) : zero;
+        C0[r] = cadd(gn, gs);
+        C1[r] = csub(gn, gs);
       } else {
-        const long rowp = (long)(L + m) * a.sm, rowm = (long)(L - m) * a.sm;
-        P0[r] = a.G[rowp + (long)rn * a.sr];
-        P1[r] = rs >= 0 ? a.G[rowp + (long)rs * a.sr] : double2{0.0, 0.0};
-        Q0[r] = cconj(a.G[rowm + (long)rn * a.sr]);
-        Q1[r] = rs >= 0 ? cconj(a.G[rowm + (long)rs * a.sr]) : double2{0.0, 0.0};
-        P1[r] = double2{sgA * P1[r].x, sgA * P1[r].y};
-        Q1[r] = double2{sgA * Q1[r].x, sgA * Q1[r].y};
+        const double2* gp = a.G + (long)(L + m) * a.sm;
+        const double2* gm = a.G + (long)(L - m) * a.sm;
+        const double2 pn = gp[(long)rn * a.sr], qn = cconj(gm[(long)rn * a.sr]);
+        const double2 ps = rs >= 0 ? cscale(gp[(long)rs * a.sr], sgA) : zero;
+        const double2 qs = rs >= 0 ? cscale(cconj(gm[(long)rs * a.sr]), sgA) : zero;
+        if constexpr (MODE == kFull) {
+          C0[r] = pn; C1[r] = ps; C2[r] = qn; C3[r] = qs;
+        } else {
+          const double ss = (a.s & 1) ? -1.0 : 1.0;
+          C0[r] = cadd(cscale(pn, ss), qs);
+          C1[r] = csub(cscale(pn, ss), qs);
+          C2[r] = cadd(qn, cscale(ps, ss));
+          C3[r] = csub(qn, cscale(ps, ss));
+        }
       }
     }
   }
-  // A group that never contributes (start past lmax) is emptied, so that the branch-free chunks below may
-  // carry it along; lall is the l from which every other group of the wave has joined.
-  int lall = l0;
+  lc = __builtin_amdgcn_readfirstlane(lc);
+  lall = __builtin_amdgcn_readfirstlane(lall);
+  if (lc > L) return;
+
+  // where this lane's total goes (one lane of each quad writes)
+  const int wl = (lane >> 2) / NA, wc = (lane >> 2) % NA;
+  const bool writer = (lane & 3) == 0;
+  const long nalm = (long)(L + 1) * (L + 2) / 2;
+  double* __restrict__ out = reinterpret_cast<double*>(
+      a.alm + (long)m * (2 * L + 1 - m) / 2 + l0 + wl + (wc >> 1) * nalm) + (wc & 1);
+
+  // One chunk of 8 l.  SLOW: a group may join, some lane may be below range; FULL: all 8 l <= L.
+  auto chunk = [&](int l, double rc, auto slow_tag, auto full_tag) {
+    constexpr bool SLOW = decltype(slow_tag)::value;
+    constexpr bool FULL = decltype(full_tag)::value;
+    double fu[R], fv[R];
+    if constexpr (SLOW) {
 #pragma unroll
-  for (int r = 0; r < kAdjR; ++r) {
-    if (lst[r] > L) {
-      x[r] = mu[r] = pm[r] = ku[r] = nv_[r] = pv[r] = kv[r] = 0.0;
-      P0[r] = P1[r] = Q0[r] = Q1[r] = double2{0.0, 0.0};
-    } else {
-      lall = max(lall, lst[r]);
+      for (int r = 0; r < R; ++r) {
+        if (l == lst[r]) {
+          const int slot = (sb * R + r) * 64 + lane;
+          if (slot < a.nslot) {
+            const long q = (long)m * a.sstride + slot;
+            const double2 sm = a.st_mu[q], sp = a.st_p[q], sk = a.st_k[q];
+            mu[r] = sm.x; pm[r] = sp.x; ku[r] = (float)sk.x;
+            if (SP) { nv[r] = sm.y; pv[r] = sp.y; kv[r] = (float)sk.y; }
+          }
+        }
+        fu[r] = rescaled_weight(mu[r], pm[r], ku[r]);
+        fv[r] = SP ? rescaled_weight(nv[r], pv[r], kv[r]) : 0.0;
+      }
     }
-  }
-  // One chunk of K l values.  FAST: every group has joined, no lane is in the scaled range and every l of the
-  // chunk is below lmax, so the chunk runs without branches; otherwise each group, scale and bound is checked.
-  auto chunk = [&](int lc, auto fast_tag) {
-    constexpr bool FAST = decltype(fast_tag)::value;
-    double2 X[K], Y[K];
+    static_for<0, CH / K>([&](auto hc) {
+      constexpr int h = decltype(hc)::value;
+      double v[16];
+      static_for<0, K>([&](auto ic) {
+        constexpr int i = decltype(ic)::value, li = h * K + i;
+        constexpr bool odd = (i & 1) != 0;
+        const double ra = row_bcast<2 * li>(rc), rb = SP ? row_bcast<2 * li + 1>(rc) : 0.0;
+        double2 X{0.0, 0.0}, Y{0.0, 0.0};
 #pragma unroll
-    for (int i = 0; i < K; ++i) X[i] = double2{0.0, 0.0};
-#pragma unroll
-    for (int i = 0; i < K; ++i) Y[i] = double2{0.0, 0.0};
-    bool slow = false;
-    bool act[kAdjR];
-#pragma unroll
-    for (int r = 0; r < kAdjR; ++r) {
-      act[r] = FAST || lc >= lst[r];
-      if (!FAST) slow |= act[r] && ((ku[r] < 0.0) || (kv[r] < 0.0));
-    }
-    if (!FAST) slow = __any(slow);
-#pragma unroll
-    for (int i = 0; i < K; ++i) {
-      const int l = lc + i;
-      if (FAST || l <= L) {
-        const double2 rc = (FAST || l < L) ? rec[l - l0] : double2{0.0, 0.0};
-#pragma unroll
-        for (int r = 0; r < kAdjR; ++r) {
-          if (!act[r]) continue;
-          double wu = mu[r], wv = nv_[r];
-          if (!FAST && slow) { wu = ku[r] == 0.0 ? wu : 0.0; wv = kv[r] == 0.0 ? wv : 0.0; }
-          if (!SP) {
-            fma2(X[i], (i & 1) ? P1[r] : P0[r], wu);
+        for (int r = 0; r < R; ++r) {
+          double wu = mu[r], wv = nv[r];
+          if (SLOW) { wu *= fu[r]; if (SP) wv *= fv[r]; }
+          if constexpr (MODE == kFull) {
+            fma2(X, C0[r], wu);
+            fma2(Y, C2[r], wv);
+            fma2(X, C1[r], odd ? -wv : wv);
+            fma2(Y, C3[r], odd ? -wu : wu);
           } else {
-            const double sv = (i & 1) ? -wv : wv, su = (i & 1) ? -wu : wu;  // sign is a compile-time constant
-            fma2(X[i], P0[r], wu);
-            fma2(X[i], P1[r], sv);
-            fma2(Y[i], Q0[r], wv);
-            fma2(Y[i], Q1[r], su);
+            fma2(X, odd ? C1[r] : C0[r], wu);
+            if (SP) fma2(X, odd ? C3[r] : C2[r], wv);
           }
-          if (FAST || l < L) {
-            double t = rc.x * x[r];
-            double nu = fma(t + rc.y, mu[r], -pm[r]);
-            pm[r] = mu[r]; mu[r] = nu;
-            if (SP) { double nn = fma(t - rc.y, nv_[r], -pv[r]); pv[r] = nv_[r]; nv_[r] = nn; }
-            if (!FAST && slow) {
-              if (ku[r] < 0.0 && fabs(mu[r]) > kThresh) { mu[r] *= kSmall; pm[r] *= kSmall; ku[r] += 1.0; }
-              if (SP && kv[r] < 0.0 && fabs(nv_[r]) > kThresh) { nv_[r] *= kSmall; pv[r] *= kSmall; kv[r] += 1.0; }
-            }
+          // a step past lmax reads a padded or neighbouring table entry; its result is never used
+          const double t = SP ? fma(ra, x[r], rb) : ra * x[r];
+          const double nu = fma(t, mu[r], -pm[r]);
+          pm[r] = mu[r]; mu[r] = nu;
+          if (SP) {
+            const double nn = fma(fma(ra, x[r], -rb), nv[r], -pv[r]);
+            pv[r] = nv[r]; nv[r] = nn;
           }
         }
-      }
-    }
-    double2 xs = transpose_reduce<K>(X);
-    if (writer) {
-      const int l = lc + ridx;
-      if (l <= L) {
-        atomicAdd(&lacc[(l - l0) * NA].x, xs.x);
-        atomicAdd(&lacc[(l - l0) * NA].y, xs.y);
-      }
-    }
-    if constexpr (SP) {
-      double2 ys = transpose_reduce<K>(Y);
-      if (writer) {
-        const int l = lc + ridx;
-        if (l <= L) {
-          atomicAdd(&lacc[(l - l0) * NA + 1].x, ys.x);
-          atomicAdd(&lacc[(l - l0) * NA + 1].y, ys.y);
-        }
-      }
-    }
+        v[i * NA] = X.x;
+        v[i * NA + 1] = X.y;
+        if constexpr (MODE == kFull) { v[i * NA + 2] = Y.x; v[i * NA + 3] = Y.y; }
+      });
+      const double total = wave_sums(v);
+      const int lh = l + h * K;
+      if (writer && (FULL || lh + wl <= L)) atomicAdd(out + 2 * (lh - l0), total);
+    });
+  };
+  auto any_under = [&]() {
+    bool under = false;
+#pragma unroll
+    for (int r = 0; r < R; ++r) under |= (ku[r] < 0.f) || (kv[r] < 0.f);
+    return __any(under);
   };
   using T_ = std::true_type;
   using F_ = std::false_type;
-  // group starts are l0 plus multiples of 8, so they fall on chunk boundaries; a lane leaves the scaled range
-  // for good once its value is unscaled, so the checked phase ends at the first chunk that qualifies
-  int lc = lmin;
-  for (; lc <= L; lc += K) {
-    bool scaled = false;
-#pragma unroll
-    for (int r = 0; r < kAdjR; ++r) scaled |= (ku[r] < 0.0) || (kv[r] < 0.0);
-    if (lc >= lall && lc + K - 1 < L && !__any(scaled)) break;
-    chunk(lc, F_{});
+  auto load = [&](int l) { return rec[2 * (long)(l - l0)]; };
+  double b0 = load(lc), b1 = load(lc + CH);
+  while (lc <= L && (lc <= lall || any_under())) {
+    const double b2 = load(lc + 2 * CH);
+    if (lc + CH - 1 <= L) chunk(lc, b0, T_{}, T_{});
+    else chunk(lc, b0, T_{}, F_{});
+    b0 = b1;
+    b1 = b2;
+    lc += CH;
   }
-  for (; lc + K - 1 < L; lc += K) chunk(lc, T_{});
-  for (; lc <= L; lc += K) chunk(lc, F_{});
-  }  // pass
-  __syncthreads();
+  while (lc + 2 * CH - 1 <= L) {
+    chunk(lc, b0, F_{}, T_{});
+    b0 = load(lc + 2 * CH);
+    chunk(lc + CH, b1, F_{}, T_{});
+    b1 = load(lc + 3 * CH);
+    lc += 2 * CH;
+  }
+  if (lc + CH - 1 <= L) {
+    chunk(lc, b0, F_{}, T_{});
+    b0 = b1;
+    lc += CH;
+  }
+  if (lc <= L) chunk(lc, b0, F_{}, F_{});
+}
 
-  // write out (also zeros for m <= l < l0)
-  const double sgs = (a.s & 1) ? -1.0 : 1.0;
-  for (int l = m + threadIdx.x; l <= L; l += blockDim.x) {
-    double2 e{0.0, 0.0}, bb{0.0, 0.0};
-    if (l >= l0) {
-      const double c = a.cnorm[base + (l - l0)];
-      if (!SP) {
-        e = lacc[l - l0];
-        e = double2{c * e.x, m == 0 ? 0.0 : c * e.y};
+__global__ void k_adjoint_clear(double2* __restrict__ p, long n) {
+  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
+    p[i] = double2{0.0, 0.0};
+}
+
+// The sums of k_adjoint -> alm, in place.  Block row y serves m = y and m = lmax - y, which together have lmax + 2 l.
+template <int MODE>
+__global__ __launch_bounds__(256) void k_adjoint_finish(int L, int s, const long* __restrict__ mofs,
+                                                        const double* __restrict__ cnorm, double2* __restrict__ alm) {
+  const long nalm = (long)(L + 1) * (L + 2) / 2;
+  for (int pass = 0; pass < 2; ++pass) {
+    const int m = pass == 0 ? (int)blockIdx.y : L - (int)blockIdx.y;
+    if (pass == 1 && m <= (int)blockIdx.y) break;  // the middle m has no partner
+    const int l0 = l0_of(m, s);
+    const long mbase = (long)m * (2 * L + 1 - m) / 2;
+    for (int l = l0 + blockIdx.x * blockDim.x + threadIdx.x; l <= L; l += gridDim.x * blockDim.x) {
+      const double c = cnorm[mofs[m] + (l - l0)];
+      double2* e = alm + mbase + l;
+      if constexpr (MODE == kScalar) {
+        *e = double2{c * e->x, m == 0 ? 0.0 : c * e->y};
+      } else if constexpr (MODE == kGrad) {
+        *e = cscale(*e, -0.5 * c);
       } else {
-        double2 X = lacc[(l - l0) * 2], Y = lacc[(l - l0) * 2 + 1];
-        X = double2{sgs * c * X.x, sgs * c * X.y};
-        Y = double2{c * Y.x, c * Y.y};
-        e = double2{-0.5 * (X.x + Y.x), -0.5 * (X.y + Y.y)};
-        bb = double2{-0.5 * (X.y - Y.y), 0.5 * (X.x - Y.x)};
+        const double sc = (s & 1) ? -c : c;
+        const double2 X = cscale(*e, sc), Y = cscale(e[nalm], c);
+        *e = double2{-0.5 * (X.x + Y.x), -0.5 * (X.y + Y.y)};
+        e[nalm] = double2{-0.5 * (X.y - Y.y), 0.5 * (X.x - Y.x)};
       }
     }
-    a.alm[mbase + l] = e;
-    if (SP && a.ncomp > 1) a.alm[nalm + mbase + l] = bb;
   }
 }
 
@@ -1377,10 +1335,10 @@ static void launch_synth(const SynthArgs& a, int variant, hipStream_t st) {
   if constexpr (NB > 1) {
     hipLaunchKernelGGL((k_synth<SP, NB, 1, 2, GR, 1>), blocks(1, 1), dim3(64), 0, st, b);
   } else if (variant == 0) {
-    constexpr int MODE = !SP ? kRowScalar : GR ? kRowGrad : kRowFull;
+    constexpr int MODE = !SP ? kScalar : GR ? kGrad : kFull;
     const dim3 grid = blocks(1, SP ? 2 : 1);
     hipLaunchKernelGGL(k_synth_row<MODE>, grid, dim3(64), 0, st, b);
-  } else if (SP) {
+  } else if constexpr (SP) {
     const dim3 grid = blocks(variant, 1);
     if (variant == 1) hipLaunchKernelGGL((k_synth<SP, 1, 1, 2, GR, 8>), grid, dim3(64), 0, st, b);
     else hipLaunchKernelGGL((k_synth<SP, 1, 2, 2, GR, 6>), grid, dim3(64), 0, st, b);
@@ -1602,38 +1560,49 @@ void legendre_autotune(LegendreTables& t, int ncomp, double2* coef_ws, double2* 
   cache[key] = {bestv, best / 2};
 }
 
+// Waves of a launch with three ring groups each from which the adjoint takes three groups per wave: below it a SIMD
+// has one or two waves, and the shorter l-step of one group is worth more than the shared lane sums.  Measured, ms, one /
+// three groups: lmax 700 spin 0 0.090 / 0.096, spin 2 0.167 / 0.174 (1402 waves); lmax 850 0.120 / 0.122, 0.224 / 0.231
+// (2553); lmax 1000 0.170 / 0.148, 0.296 / 0.276 (3003).
+constexpr long kAdjointMinWaves = 2600;
+
+template <int MODE>
+static void launch_adjoint(const LegendreTables& t, AdjArgs a, hipStream_t st) {
+  const int L = t.lmax;
+  const long n = (long)(L + 1) * (L + 2) / 2 * (MODE == kFull ? 2 : 1);
+  hipLaunchKernelGGL(k_adjoint_clear, dim3((unsigned)std::min<long>(4096, (n + 255) / 256)), dim3(256), 0, st, a.alm, n);
+  NUSHT_LAUNCH_CHECK();
+  const int R = (long)(L + 1) * ceil_div(t.ngroups, 3) < kAdjointMinWaves ? 1 : 3;
+  a.nsb = ceil_div(t.ngroups, R) | 1;  // odd, as in launch_synth
+  const dim3 grid((unsigned)(a.nsb * ceil_div(L + 1, kNumXcd) * kNumXcd));
+  if (R == 1) hipLaunchKernelGGL((k_adjoint<MODE, 1>), grid, dim3(64), 0, st, a);
+  else hipLaunchKernelGGL((k_adjoint<MODE, 3>), grid, dim3(64), 0, st, a);
+  NUSHT_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_adjoint_finish<MODE>, dim3(ceil_div(L + 1, 1024), L / 2 + 1), dim3(256), 0, st, L, t.spin,
+                     t.mofs.as<long>(), t.cnorm.as<double>(), a.alm);
+  NUSHT_LAUNCH_CHECK();
+}
+
 void legendre_adjoint(const LegendreTables& t, int ncomp, const double2* G, long sm, long sr, double2* alm,
                       hipStream_t st) {
-  const int L = t.lmax;
   AdjArgs a;
-  a.lmax = L; a.s = t.spin; a.nslot = t.nslot; a.sstride = t.sstride; a.ngroups = t.ngroups; a.ncomp = ncomp;
+  a.lmax = t.lmax; a.s = t.spin; a.nslot = t.nslot; a.sstride = t.sstride; a.ngroups = t.ngroups; a.nsb = 0;
   a.slot_theta = t.slot_theta.as<double>();
   a.slot_north = t.slot_north.as<int>();
   a.slot_south = t.slot_south.as<int>();
   a.mofs = t.mofs.as<long>();
   a.rec = t.rec.as<double2>();
-  a.cnorm = t.cnorm.as<double>();
   a.st_mu = t.st_mu.as<double2>();
   a.st_p = t.st_p.as<double2>();
   a.st_k = t.st_k.as<double2>();
   a.start = t.start.as<int>();
   a.G = G; a.sm = sm; a.sr = sr; a.alm = alm;
-  const int R = t.spin ? AdjCfg<true>::R : AdjCfg<false>::R;
-  const int maxw = (t.spin ? AdjCfg<true>::MaxThreads : AdjCfg<false>::MaxThreads) / 64;
-  int nw = std::min(maxw, ceil_div(t.nslot, 64 * R));  // more rings run as further passes
-  if (nw < 1) nw = 1;
-  const int na = t.spin ? 2 : 1;
-  const size_t lds = sizeof(double2) * (size_t)(L + 1) * na;
-  NUSHT_REQUIRE(lds <= 160 * 1024, kErrUnsupported, "legendre_adjoint: lmax too large for the LDS accumulator");
+  // the lmax that the adjoint is built and checked for
+  NUSHT_REQUIRE(t.lmax <= (t.spin ? 5119 : 10239), kErrUnsupported, "legendre_adjoint: lmax too large");
   StageScope sc(t.n_adj.c_str(), st);
-  if (t.spin) {
-    NUSHT_HIP(hipFuncSetAttribute((const void*)k_adjoint<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(k_adjoint<true>, dim3(L + 1), dim3(64 * nw), lds, st, a);
-  } else {
-    NUSHT_HIP(hipFuncSetAttribute((const void*)k_adjoint<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(k_adjoint<false>, dim3(L + 1), dim3(64 * nw), lds, st, a);
-  }
-  NUSHT_LAUNCH_CHECK();
+  if (t.spin == 0) launch_adjoint<kScalar>(t, a, st);
+  else if (ncomp == 1) launch_adjoint<kGrad>(t, a, st);
+  else launch_adjoint<kFull>(t, a, st);
 }
 
 }  // namespace nusht
