@@ -47,7 +47,7 @@ struct NufftParams {
 // Precomputed tables and per-plan buffers.
 class NufftPlan {
  public:
-  // tile_rows: rows of the register row-window spreading tiles (0: 8, or NUSHT_SPREAD_TR)
+  // tile_rows: rows of the windowed spreading tiles (0: 8, or NUSHT_SPREAD_TR)
   NufftPlan(const NufftParams& p, long npts_max, hipStream_t st, int tile_rows = 0);
   int tile_rows() const { return tile_r_; }
   int tile_cols() const { return tile_c_; }
@@ -82,7 +82,7 @@ class NufftPlan {
   long npts_max_ = 0;
   long npts_ = 0;
   int tile_r_ = 32, tile_c_ = 32;  // spreading tile (fine cells)
-  bool rows_spread_ = false;       // register row-window spreading (8 <= w <= 16)
+  bool rows_spread_ = false;       // windowed spreading: matrix cores (w 8..13) or row windows (14..16)
   int rows_cap_ = 0;               // its LDS point records per pass
   int rows_seg_ = 1;               // tiles one workgroup walks down a column strip
   int ntile_r_ = 0, ntile_c_ = 0;
@@ -106,7 +106,7 @@ class NufftPlan {
 
 // Plan-time choice of the fine-grid oversampling sigma and the spreading tile height by measurement: every
 // candidate (sigma in {1.25, 1.5, 2} and the default rule, as far as the fine grid fits the in-LDS
-// transforms; tile heights 8, 16, 32 where the register row-window spreading applies) is built and timed on
+// transforms; tile heights 8, 16, 32 where the windowed spreading applies) is built and timed on
 // npts_max synthetic points (theta = acos U(-1, 1), phi = U(0, 2 pi)) for one type-2 and one type-1
 // transform from / into G (rows m with stride g_stride_m; contents are overwritten); the plan with the
 // least type-2 + type-1 time is returned.  Results are cached per (device, lmax, spin, eps, npts_max).

@@ -742,7 +742,9 @@ __global__ __launch_bounds__(256) void k_spread_w(SpreadArgs<T> a) {
 constexpr int kMaxUnrolledW = 16;
 
 // ------------------------------------------------------------------ spreading by register row windows
-// Widths kRowsMinW..kRowsMaxW.  A tile is tr rows x 16 SW columns of first cells (i0, j0), SW = 17 - W:
+// Widths kMmMaxW + 1 .. kRowsMaxW (the matrix-core spreading below takes the narrower ones: its windows would be three
+// cells wide or less here, too few points for its groups of four).  A tile is tr rows x 16 SW columns of first cells
+// (i0, j0), SW = 17 - W:
 // 16-lane group g owns the 16 fine columns [g SW, g SW + 16) of the tile (+ halo), which hold the whole
 // W-column footprint of every point whose first column lies in the group's slice [g SW, g SW + SW).  The
 // points of the tile are counting-sorted in LDS by (slice, first row); each group then walks the rows
@@ -758,6 +760,7 @@ constexpr int kMaxUnrolledW = 16;
 // ring, so the W - 1 halo rows below a tile carry over to the next instead of going to HBM with atomics.
 constexpr int kRowsMinW = 8;
 constexpr int kRowsMaxW = 16;
+constexpr int kMmMaxW = 13;      // widths up to here spread on the matrix cores
 constexpr int kRowsGroups = 16;  // 16-lane groups per 256-thread workgroup (= slices per tile)
 constexpr int kRowsPts = 3;      // points per thread in one pass of the row-window spreading (records <= 768)
 constexpr int kRowsMinDeg = 3;   // kernel polynomial degrees with a register-resident Horner
@@ -836,7 +839,7 @@ __host__ __device__ inline RowsLayout rows_layout(int w, int tr, int deg, int ca
 
 template <typename T, int W, int DM>
 __global__ __launch_bounds__(256) void k_spread_rows(SpreadArgs<T> a, RowsLayout lay) {
-  static_assert(W >= kRowsMinW && W <= kRowsMaxW, "register row windows for 8 <= W <= 16");
+  static_assert(W > kMmMaxW && W <= kRowsMaxW, "register row windows for 14 <= W <= 16");
   constexpr int SW = 17 - W;
   using T2 = c2_t<T>;
   extern __shared__ unsigned char smem_raw[];
@@ -1045,6 +1048,289 @@ __global__ __launch_bounds__(256) void k_spread_rows(SpreadArgs<T> a, RowsLayout
   // rows r0 .. r0 + tr - 1 get nothing from later tiles of the strip
   flush_rows(r0, base, 0, tr);
   __syncthreads();
+  }
+  // the W - 1 rows below the last tile are shared with the next segment
+  flush_rows((t1 - 1) * tr, ((t1 - 1 - t0) * tr) % R, tr, R);
+}
+
+// ------------------------------------------------------------------ spreading on the matrix cores
+// Widths kRowsMinW..kMmMaxW, on the tiles and column strips of the row windows.  Points whose first cell lies in one
+// window of RS rows x SW columns (RS = 4, or 8 for w <= 9) have their whole footprint in the 16 x 16 cells from the
+// window's first cell on, so the window receives a matrix product: 16 rows x points of row weights times
+// points x 16 columns of value times column weight, four points per v_mfma_f64_16x16x4_f64 (one for the real and one
+// for the imaginary part).  The tile's points are counting-sorted in LDS by (column window, row step), each window's
+// records padded to a multiple of four with zero values.  A wave takes a column window and steps down its rows: each
+// lane evaluates the kernel polynomial of cell l16 along both axes for its 16-lane row's point (the coefficients stay
+// in registers, zero above the degree) and the two weights are rotated inside the row by the point's offsets in the
+// window, cells past the width being zero; the finished RS rows of the accumulator go to the LDS ring (ds_add_f64:
+// neighbouring windows overlap) and the registers move up by RS rows, four rows each.
+// What bounds it: issue.  Per four points (3.6 after padding at 0.64 points per cell, w = 12) two MFMAs take 130
+// cycles and about 45 VALU instructions 190; the row windows spent as much on the contraction and waited for the
+// busiest of four 16-lane groups besides (1.6 times the mean).  Walk 1.55 of 2.28 ms at lmax 4095 (eps 1e-7, w = 12,
+// 33.5M points; two waves per SIMD and register copies around each MFMA if the accumulators go to AGPRs, hence the
+// waves-per-EU attribute: 2.55 ms).  Before, by row windows, and now, ms: lmax 4095 3.22 -> 2.28, lmax 3001 2.44 ->
+// 1.55, lmax 2047 eps 1e-10 (w = 11, 8.4M points) 1.56 -> 1.06.  Tile heights 4 / 8 / 12 / 16 rows at lmax 4095:
+// 2.58 / 2.28 / 2.57 / 2.90.
+// Operand layouts of v_mfma_f64_16x16x4_f64: A[i][k] in lane i + 16 k, B[k][j] in lane j + 16 k, D[i][j] in register
+// i / 4 of lane j + 16 (i % 4).
+struct MmLayout {
+  int tr, tc, aw, cap, deg, nstep, nkey;
+  int seg, ntr;  // as in RowsLayout
+  size_t re_off, im_off, val_off, uu_off, off_off, cnt_off, bytes;
+};
+
+template <typename T>
+__host__ __device__ inline MmLayout mm_layout(int w, int tr, int deg, int cap) {
+  MmLayout L;
+  const int sw = 17 - w, rs = w <= 9 ? 8 : 4;
+  L.tr = tr;
+  L.tc = kRowsGroups * sw;
+  L.aw = L.tc + w - 1;
+  L.cap = cap;
+  L.deg = deg;
+  L.nstep = (tr + rs - 1) / rs;
+  L.nkey = kRowsGroups * L.nstep;
+  L.seg = 1;
+  L.ntr = 0;
+  const size_t plane = sizeof(double) * (size_t)(tr + w - 1) * L.aw;
+  size_t o = 0;
+  L.re_off = o; o += plane;
+  L.im_off = o; o += plane;
+  o = (o + 15) & ~(size_t)15;
+  // each window's records are padded to a multiple of 4, and the walk reads two groups of 4 ahead
+  const size_t nrec = (size_t)cap + 3 * L.nkey + 8;
+  L.val_off = o; o += sizeof(double2) * nrec;
+  L.uu_off = o;  o += sizeof(c2_t<T>) * nrec;
+  L.off_off = o; o += nrec;
+  o = (o + 15) & ~(size_t)15;
+  L.cnt_off = o; o += sizeof(int) * (size_t)(2 * L.nkey + 1);
+  L.bytes = o;
+  return L;
+}
+
+typedef double v4d_t __attribute__((ext_vector_type(4)));
+
+// the value of lane `src` (byte address of a lane: 4 * lane)
+__device__ __forceinline__ double lane_read(double v, int src4) {
+  return __hiloint2double(__builtin_amdgcn_ds_bpermute(src4, __double2hiint(v)),
+                          __builtin_amdgcn_ds_bpermute(src4, __double2loint(v)));
+}
+__device__ __forceinline__ float lane_read(float v, int src4) {
+  return __int_as_float(__builtin_amdgcn_ds_bpermute(src4, __float_as_int(v)));
+}
+
+template <typename T, int W, int DM>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DM <= 12 ? 3 : 2))) void k_spread_mm(SpreadArgs<T> a, MmLayout lay) {
+  static_assert(W >= kRowsMinW && W <= kMmMaxW, "16 x 16 windows of at least 4 x 4 first cells");
+  constexpr int SW = 17 - W;
+  constexpr int RS = W <= 9 ? 8 : 4, NR = RS / 4;  // rows and registers per step
+  using T2 = c2_t<T>;
+  extern __shared__ unsigned char smem_raw[];
+  double* acc_re = reinterpret_cast<double*>(smem_raw + lay.re_off);  // (tr + W - 1) x aw each
+  double* acc_im = reinterpret_cast<double*>(smem_raw + lay.im_off);
+  double2* val = reinterpret_cast<double2*>(smem_raw + lay.val_off);  // rotated value per point record
+  T2* uu = reinterpret_cast<T2*>(smem_raw + lay.uu_off);               // its row and column polynomial arguments
+  unsigned char* offs = smem_raw + lay.off_off;                        // its first row and column in the window
+  int* cnt = reinterpret_cast<int*>(smem_raw + lay.cnt_off);  // [nkey]: counts, then cursors
+  int* start = cnt + lay.nkey;                                 // [nkey + 1]
+  const int tile_c = blockIdx.x % a.ntc;
+  const int t0 = (blockIdx.x / a.ntc) * lay.seg, t1 = min(t0 + lay.seg, lay.ntr);
+  if (a.tile_start[t0 * a.ntc + tile_c] == a.tile_start[(t1 - 1) * a.ntc + tile_c + 1]) return;  // no points
+  const int tr = lay.tr, aw = lay.aw, nkey = lay.nkey, nstep = lay.nstep;
+  const int R = tr + W - 1;
+  for (int i = threadIdx.x; i < R * aw; i += blockDim.x) acc_re[i] = acc_im[i] = 0.0;
+  __syncthreads();
+  const int c0 = tile_c * a.tc;
+  // cells no other workgroup touches, as in k_spread_rows
+  const int excl_c1 = a.ntc >= 2 ? min(a.tc, a.nf - c0) : 0;
+  const int excl_r0 = t0 == 0 ? 0 : t0 * tr + W - 1, excl_r1 = t1 * tr;
+  const double scale = a.nf / (2.0 * M_PI);
+  const double hw = 0.5 * W;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int l16 = lane & 15, q16 = lane >> 4;
+  T cf[DM + 1];
+#pragma unroll
+  for (int k = 0; k <= DM; ++k) cf[k] = (l16 < W && k <= lay.deg) ? a.kpoly[(long)k * W + l16] : T(0);
+  auto cells = [&](int p, int r0, int& lr, int& lc, double& ut, double& up, int& i0, int& j0u) {
+    const double2 tp = a.pts[p];
+    ut = tp.x * scale;
+    up = tp.y * scale;
+    up -= a.nf * floor(up / a.nf);
+    i0 = (int)ceil(ut - hw);
+    j0u = (int)ceil(up - hw);
+    const int j0 = j0u < 0 ? j0u + a.nf : j0u;
+    lr = i0 - a.row_lo - r0;
+    lc = j0 - c0;
+  };
+  auto flush_rows = [&](int r0, int base, int rb, int re) {
+    for (int i = threadIdx.x; i < (re - rb) * aw; i += blockDim.x) {
+      const int rr = rb + i / aw, cc = i % aw;
+      int slot = base + rr;  // base < R, rr < R
+      slot -= slot >= R ? R : 0;
+      const int cell = slot * aw + cc;
+      const T vr = (T)acc_re[cell], vi = (T)acc_im[cell];
+      acc_re[cell] = acc_im[cell] = 0.0;
+      const int grow = r0 + rr;
+      if (grow >= a.nrow) continue;
+      if (vr == T(0) && vi == T(0)) continue;
+      const int gc = (c0 + cc) % a.nf;  // a strip can be wider than a small grid
+      T* g = reinterpret_cast<T*>(a.grid + (long)grow * a.nf + gc);
+      if (grow >= excl_r0 && grow < excl_r1 && cc >= W - 1 && cc < excl_c1) {
+        *reinterpret_cast<c2_t<T>*>(g) = c2_t<T>{vr, vi};
+      } else {
+        atomicAdd(&g[0], vr);
+        atomicAdd(&g[1], vi);
+      }
+    }
+  };
+  for (int t = t0; t < t1; ++t) {
+    const int tb = t * a.ntc + tile_c;
+    const int s0 = a.tile_start[tb], s1 = a.tile_start[tb + 1];
+    const int r0 = t * tr;
+    const int base = ((t - t0) * tr) % R;  // ring slot of the tile's first row
+    for (int cb = s0; cb < s1; cb += lay.cap) {
+      const int n = min(lay.cap, s1 - cb);
+      for (int i = threadIdx.x; i < nkey; i += blockDim.x) cnt[i] = 0;
+      __syncthreads();
+      // pass 1: each thread holds up to kRowsPts points of the pass: key, polynomial arguments, offsets and (rotated)
+      // value, whose gathers are in flight across the count and the scan
+      int keyv[kRowsPts], offv[kRowsPts];
+      T2 uuv[kRowsPts];
+      double vrv[kRowsPts], viv[kRowsPts];
+#pragma unroll
+      for (int k = 0; k < kRowsPts; ++k) {
+        const int q = threadIdx.x + k * 256;
+        keyv[k] = -1;
+        offv[k] = 0;
+        uuv[k] = T2{T(0), T(0)};
+        vrv[k] = viv[k] = 0.0;
+        if (q < n) {
+          const int p = cb + q;
+          int lr, lc, i0, j0u;
+          double ut, up;
+          cells(p, r0, lr, lc, ut, up, i0, j0u);
+          if (lr >= 0 && lr < tr && lc >= 0 && lc < lay.tc) {  // always, for points binned by set_pts
+            keyv[k] = (lc / SW) * nstep + lr / RS;
+            offv[k] = (lr % RS) * 16 + lc % SW;
+            uuv[k] = T2{(T)((i0 - ut) + 0.5 * W - 0.5), (T)((j0u - up) + 0.5 * W - 0.5)};
+            const int o = a.idx[p];
+            vrv[k] = a.in_re[o];
+            viv[k] = (a.spin && a.in_im) ? a.in_im[o] : 0.0;
+            if (a.spin && a.gamma) {
+              double sn, cs;
+              sincos(-a.spin * a.gamma[o], &sn, &cs);
+              const double xr = vrv[k] * cs - viv[k] * sn, xi = vrv[k] * sn + viv[k] * cs;
+              vrv[k] = xr;
+              viv[k] = xi;
+            }
+            atomicAdd(&cnt[keyv[k]], 1);
+          }
+        }
+      }
+      __syncthreads();
+      // exclusive scan of the padded counts (one wave, nkey <= 16 x 8)
+      if (wave == 0) {
+        const int per = (nkey + 63) / 64;
+        int sum = 0;
+        for (int i = 0; i < per; ++i) {
+          const int k = lane * per + i;
+          sum += k < nkey ? (cnt[k] + 3) & ~3 : 0;
+        }
+        int incl = sum;
+        for (int d = 1; d < 64; d <<= 1) {
+          const int u = __shfl_up(incl, d, 64);
+          if (lane >= d) incl += u;
+        }
+        int run = incl - sum;
+        for (int i = 0; i < per; ++i) {
+          const int k = lane * per + i;
+          if (k < nkey) {
+            start[k] = run;
+            run += (cnt[k] + 3) & ~3;
+          }
+        }
+        if (lane == 63) start[nkey] = incl;
+      }
+      __syncthreads();
+      for (int k = threadIdx.x; k < nkey; k += blockDim.x)  // the padding records add nothing
+        for (int pos = start[k] + cnt[k]; pos < start[k + 1]; ++pos) {
+          val[pos] = double2{0.0, 0.0};
+          uu[pos] = T2{T(0), T(0)};
+          offs[pos] = 0;
+        }
+      __syncthreads();
+      // pass 2: records in sorted order (cnt counts down as the cursor)
+#pragma unroll
+      for (int k = 0; k < kRowsPts; ++k) {
+        if (keyv[k] < 0) continue;
+        const int pos = start[keyv[k]] + atomicSub(&cnt[keyv[k]], 1) - 1;
+        val[pos] = double2{vrv[k], viv[k]};
+        uu[pos] = uuv[k];
+        offs[pos] = (unsigned char)offv[k];
+      }
+      __syncthreads();
+      for (int cw = wave; cw < kRowsGroups; cw += 4) {
+        // groups of 4 records of the column window, in row-step order
+        const int kb = cw * nstep;
+        int g = __builtin_amdgcn_readfirstlane(start[kb]) >> 2;
+        const int gend = __builtin_amdgcn_readfirstlane(start[kb + nstep]) >> 2;
+        if (g == gend) continue;  // no points
+        int rs = 0, gstep = __builtin_amdgcn_readfirstlane(start[kb + 1]) >> 2;  // row step and the end of its groups
+        v4d_t dr{0.0, 0.0, 0.0, 0.0}, di{0.0, 0.0, 0.0, 0.0};
+        const int acol = cw * SW + l16;
+        auto add_rows = [&](int row, double vr, double vi) {  // row: of this lane, relative to the tile
+          if (row < R) {
+            int slot = base + row;
+            slot -= slot >= R ? R : 0;
+            atomicAdd(&acc_re[slot * aw + acol], vr);
+            atomicAdd(&acc_im[slot * aw + acol], vi);
+          }
+        };
+        auto end_step = [&]() {  // rows rs RS .. rs RS + RS - 1 are complete
+#pragma unroll
+          for (int i = 0; i < NR; ++i) add_rows(rs * RS + 4 * i + q16, dr[i], di[i]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            dr[i] = i + NR < 4 ? dr[(i + NR) & 3] : 0.0;
+            di[i] = i + NR < 4 ? di[(i + NR) & 3] : 0.0;
+          }
+          ++rs;
+        };
+        // The records of group g + 2 are read, and the weights of group g + 1 evaluated, while the weights of group g
+        // rotate through the LDS lane exchange.
+        struct Rec {
+          double2 v;
+          T2 u;
+          int off;
+        };
+        auto record = [&](int gg) { return Rec{val[4 * gg + q16], uu[4 * gg + q16], offs[4 * gg + q16]}; };
+        Rec r0 = record(g), r1 = record(g + 1);
+        T kt, kp;
+        horner2<DM, DM>(cf, r0.u.x, r0.u.y, kt, kp);
+#pragma unroll 2
+        for (; g < gend; ++g) {
+          const double wt = (double)lane_read(kt, 4 * ((lane & 48) + ((l16 - (r0.off >> 4)) & 15)));
+          const double wp = (double)lane_read(kp, 4 * ((lane & 48) + ((l16 - r0.off) & 15)));
+          const Rec r2 = record(g + 2);
+          horner2<DM, DM>(cf, r1.u.x, r1.u.y, kt, kp);
+          while (g >= gstep) {
+            end_step();
+            gstep = __builtin_amdgcn_readfirstlane(start[kb + rs + 1]) >> 2;
+          }
+          dr = __builtin_amdgcn_mfma_f64_16x16x4f64(wt, r0.v.x * wp, dr, 0, 0, 0);
+          di = __builtin_amdgcn_mfma_f64_16x16x4f64(wt, r0.v.y * wp, di, 0, 0, 0);
+          r0 = r1;
+          r1 = r2;
+        }
+        while (rs < nstep) end_step();
+#pragma unroll
+        for (int i = 0; i < 4 - NR; ++i) add_rows(nstep * RS + 4 * i + q16, dr[i], di[i]);
+      }
+      __syncthreads();  // records are rewritten by the next pass
+    }
+    // rows r0 .. r0 + tr - 1 get nothing from later tiles of the strip
+    flush_rows(r0, base, 0, tr);
+    __syncthreads();
   }
   // the W - 1 rows below the last tile are shared with the next segment
   flush_rows((t1 - 1) * tr, ((t1 - 1 - t0) * tr) % R, tr, R);
@@ -1282,6 +1568,26 @@ void launch_spread_rows(int w, dim3 grid, hipStream_t st, const SpreadArgs<T>& a
   }
 }
 
+template <typename T, int W>
+void launch_spread_mm(int w, dim3 grid, hipStream_t st, const SpreadArgs<T>& a, const MmLayout& lay) {
+  if constexpr (W > kMmMaxW) {
+    throw Error{kErrUnsupported, "nufft: no matrix-core spreading for this width"};
+  } else {
+    if (w == W) {
+      // the polynomial's coefficients above its degree are zero: 8 covers eps 1e-7, 12 most of the rest
+      auto launch = [&](auto kern) {
+        NUSHT_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lay.bytes));
+        hipLaunchKernelGGL(kern, grid, dim3(256), lay.bytes, st, a, lay);
+      };
+      if (lay.deg <= 8) launch(k_spread_mm<T, W, 8>);
+      else if (lay.deg <= 12) launch(k_spread_mm<T, W, 12>);
+      else launch(k_spread_mm<T, W, 24>);
+    } else {
+      launch_spread_mm<T, W + 1>(w, grid, st, a, lay);
+    }
+  }
+}
+
 NufftParams NufftParams::choose(int lmax, int spin, double eps, double sigma_hint) {
   NUSHT_REQUIRE(lmax >= 1, kErrArg, "nufft: lmax must be >= 1");
   NUSHT_REQUIRE(eps > 0 && eps < 1, kErrArg, "nufft: epsilon must be in (0, 1)");
@@ -1437,7 +1743,7 @@ NufftPlan::NufftPlan(const NufftParams& p, long npts_max, hipStream_t st, int ti
   const size_t cb = p.single ? 8 : 16;
   T_.alloc(cb * (size_t)p.nrow * p.nm);
   grid_.alloc(cb * (size_t)p.nrow * p.nf);
-  // tiles: tile_r_ rows (default 8) x 16 (17 - w) columns for the register row-window spreading (8 <= w <= 16; the
+  // tiles: tile_r_ rows (default 8) x 16 (17 - w) columns for the windowed spreading (8 <= w <= 16; the
   // interpolation takes the same tiles), 32 x 32 otherwise.  NUSHT_SPREAD_ROWS=0 keeps the LDS-atomic
   // spreading and its tiles; NUSHT_SPREAD_TR sets the tile height (rows of first cells).
   rows_spread_ = fitted && p.w >= kRowsMinW && p.w <= kRowsMaxW && p_.poly_deg >= kRowsMinDeg &&
@@ -1453,13 +1759,16 @@ NufftPlan::NufftPlan(const NufftParams& p, long npts_max, hipStream_t st, int ti
     // workgroups per CU when 256 records fit in 52 KiB, two when they fit in 78 KiB, else one with up to
     // 156 KiB; the records left over in the chosen budget are used too (fewer passes over a tile)
     const size_t rec = sizeof(double2) + (p.single ? sizeof(float2) : sizeof(double2)) + 1;
-    const RowsLayout base = p.single ? rows_layout<float>(p.w, tr, p_.poly_deg, 0)
-                                     : rows_layout<double>(p.w, tr, p_.poly_deg, 0);
-    const size_t budget = base.bytes + 256 * rec <= 52 * 1024   ? 52 * 1024
-                          : base.bytes + 256 * rec <= 78 * 1024 ? 78 * 1024
-                                                                : 156 * 1024;
-    NUSHT_REQUIRE(base.bytes + 64 * rec <= budget, kErrUnsupported, "nufft: spreading tile too large for LDS");
-    long cap = (long)((budget - base.bytes) / rec);
+    const auto layout_bytes = [&](auto lay) { return lay.bytes; };
+    const size_t base = p.w <= kMmMaxW ? (p.single ? layout_bytes(mm_layout<float>(p.w, tr, p_.poly_deg, 0))
+                                                   : layout_bytes(mm_layout<double>(p.w, tr, p_.poly_deg, 0)))
+                                       : (p.single ? layout_bytes(rows_layout<float>(p.w, tr, p_.poly_deg, 0))
+                                                   : layout_bytes(rows_layout<double>(p.w, tr, p_.poly_deg, 0)));
+    const size_t budget = base + 256 * rec <= 52 * 1024   ? 52 * 1024
+                          : base + 256 * rec <= 78 * 1024 ? 78 * 1024
+                                                          : 156 * 1024;
+    NUSHT_REQUIRE(base + 64 * rec <= budget, kErrUnsupported, "nufft: spreading tile too large for LDS");
+    long cap = (long)((budget - base) / rec);
     cap = std::max(64L, std::min(256L * kRowsPts, cap - cap % 64));
     rows_cap_ = (int)cap;
   }
@@ -1594,11 +1903,16 @@ void NufftPlan::type1_impl(const double* ire, const double* iim, const double* g
     SpreadArgs<T> sa{p.nf, p.w, p.row_lo, p.nrow, p.spin, tile_r_, tile_c_, ntile_c_, (T)p.beta, kpoly_.as<T>(),
                      p.poly_deg, pts_.as<double2>(), idx_.as<int>(), tile_start_.as<int>(), ire, iim, gamma,
                      grid_.as<T2>()};
-    if (rows_spread_) {
+    if (rows_spread_ && p.w <= kMmMaxW) {
+      MmLayout lay = mm_layout<T>(p.w, tile_r_, p.poly_deg, rows_cap_);
+      lay.seg = rows_seg_;
+      lay.ntr = ntile_r_;
+      launch_spread_mm<T, kRowsMinW>(p.w, dim3(ntile_c_ * (int)ceil_div(ntile_r_, rows_seg_)), st, sa, lay);
+    } else if (rows_spread_) {
       RowsLayout lay = rows_layout<T>(p.w, tile_r_, p.poly_deg, rows_cap_);
       lay.seg = rows_seg_;
       lay.ntr = ntile_r_;
-      launch_spread_rows<T, kRowsMinW>(p.w, dim3(ntile_c_ * (int)ceil_div(ntile_r_, rows_seg_)), st, sa, lay);
+      launch_spread_rows<T, kMmMaxW + 1>(p.w, dim3(ntile_c_ * (int)ceil_div(ntile_r_, rows_seg_)), st, sa, lay);
     } else {
       const size_t lds = sizeof(double2) * (size_t)(tile_r_ + p.w) * (tile_c_ + p.w);  // FP64 accumulation tile
       launch_spread<T, 2>(p.w, dim3(ntile_r_ * ntile_c_), lds, st, sa);
