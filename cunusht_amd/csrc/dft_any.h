@@ -1,4 +1,4 @@
-// DFT of any length up to kDftNMAX in LDS, one workgroup of kDftNT threads per transform.
+// DFT of any length up to kDftNMAX in LDS, one workgroup (of kDftNT threads at the largest) per transform.
 //
 // Each distinct length gets a description: a direct mixed-radix FFT when n factors into 2, 3, 5,
 // 7, 13; Rader's algorithm when n is prime with a smooth n - 1; Bluestein's chirp-z algorithm when
@@ -24,7 +24,6 @@ constexpr int kDftMethods = 4;
 // and 768 rather than 640 threads halves its register spill.
 constexpr int kDftNT = 768;
 constexpr int kDftNMAX = 8320;
-constexpr int kDftE = (kDftNMAX + kDftNT - 1) / kDftNT;  // values per thread held in registers
 
 // Kernel-argument view of one length.
 template <typename T>
@@ -44,35 +43,33 @@ struct DftLen {
 
 // Forward DFT of buf[0..n) by Bluestein's algorithm on the padded length L.mlen:
 // X_k = c_k sum_j (x_j c_j) conj(c)_{k-j},  c_j = e^{-i pi j^2 / n}.
-template <typename T>
+template <typename T, int NT, int NMAX>
 __device__ __forceinline__ void bluestein_lds(c2_t<T>* buf, int n, const DftLen<T>& L) {
   using T2 = c2_t<T>;
-  constexpr int NT = kDftNT;
   const int M = L.mlen;
   for (int j = threadIdx.x; j < M; j += NT) buf[j] = j < n ? cmul(buf[j], L.chirp[j]) : T2{T(0), T(0)};
   __syncthreads();
-  fft_lds<T, NT, kDftNMAX, true>(buf, L.fd);
+  fft_lds<T, NT, NMAX, true>(buf, L.fd);
   for (int j = threadIdx.x; j < M; j += NT) buf[j] = cconj(cmul(buf[j], L.kern[j]));
   __syncthreads();
-  fft_lds<T, NT, kDftNMAX, true>(buf, L.fd);
+  fft_lds<T, NT, NMAX, true>(buf, L.fd);
   const T inv = T(1) / T(M);
   for (int k = threadIdx.x; k < n; k += NT) buf[k] = cscale(cmul(L.chirp[k], cconj(buf[k])), inv);
   __syncthreads();
 }
 
-// In-place forward DFT of buf[0..L.n) in LDS (buf holds L.lds_values() entries).  All kDftNT threads call it.
-template <int METHOD, typename T>
+// In-place forward DFT of buf[0..L.n) in LDS (buf holds L.lds_values() <= NMAX entries).  All NT threads call it.
+template <int METHOD, typename T, int NT = kDftNT, int NMAX = kDftNMAX>
 __device__ __forceinline__ void dft_lds(c2_t<T>* buf, const DftLen<T>& L) {
   using T2 = c2_t<T>;
   const int n = L.n;
-  constexpr int NT = kDftNT;
-  constexpr int E = kDftE;
+  constexpr int E = (NMAX + NT - 1) / NT;  // values per thread held in registers
   if constexpr (METHOD == (int)DftMethod::Direct) {
-    fft_lds<T, NT, kDftNMAX, true>(buf, L.fd);
+    fft_lds<T, NT, NMAX, true>(buf, L.fd);
     return;
   }
   if constexpr (METHOD == (int)DftMethod::Bluestein) {
-    bluestein_lds<T>(buf, n, L);
+    bluestein_lds<T, NT, NMAX>(buf, n, L);
     return;
   }
   if constexpr (METHOD == (int)DftMethod::Split) {
@@ -94,9 +91,9 @@ __device__ __forceinline__ void dft_lds(c2_t<T>* buf, const DftLen<T>& L) {
       }
       __syncthreads();
       if (L.sub_bluestein) {
-        bluestein_lds<T>(buf, b, L);
+        bluestein_lds<T, NT, NMAX>(buf, b, L);
       } else {
-        fft_lds<T, NT, kDftNMAX, true>(buf, L.fd);
+        fft_lds<T, NT, NMAX, true>(buf, L.fd);
       }
 #pragma unroll
       for (int i = 0; i < E; ++i) {
@@ -140,7 +137,7 @@ __device__ __forceinline__ void dft_lds(c2_t<T>* buf, const DftLen<T>& L) {
     if (q < n1) buf[q] = v[i];
   }
   __syncthreads();
-  fft_lds<T, NT, kDftNMAX, true>(buf, L.fd);
+  fft_lds<T, NT, NMAX, true>(buf, L.fd);
   const T2 a0 = buf[0];
 #pragma unroll
   for (int i = 0; i < E; ++i) v[i] = L.kern[min((int)threadIdx.x + i * NT, n1 - 1)];
@@ -151,7 +148,7 @@ __device__ __forceinline__ void dft_lds(c2_t<T>* buf, const DftLen<T>& L) {
     if (q < n1) buf[q] = cconj(cmul(buf[q], v[i]));
   }
   __syncthreads();
-  fft_lds<T, NT, kDftNMAX, true>(buf, L.fd);
+  fft_lds<T, NT, NMAX, true>(buf, L.fd);
   const T inv = T(1) / T(n1);
 #pragma unroll
   for (int i = 0; i < E; ++i) {

@@ -1846,10 +1846,17 @@ struct Pass;
 template <typename T>
 static constexpr int nmax_big() { return kLdsBytes / (int)sizeof(c2_t<T>); }
 
+// Workgroup sizes of the DFS passes by transform length.  A thread keeps eight to ten values of the row in registers
+// (92 - 128 VGPRs in FP64, four waves per SIMD), so a CU runs four 256-thread, two 512-thread or one 1024-thread
+// workgroups; several cover each other's barriers, loads and stores.
+// With 1024 threads for every length above 2048 and now, theta and phi pass: lmax 1024 FP64 (grid near 2560) 74 -> 56
+// and 70 -> 48 us, lmax 2047 FP32 (5120) 152 -> 81 and 180 -> 70 us.
 #define NUSHT_LAUNCH_SIZED(KERN, T, n, nblocks, lds, args, st)                                        \
   do {                                                                                               \
     if ((n) <= 2048) launch_pass<T, 256, 2048>(KERN<T, 256, 2048>, nblocks, lds, args, st);           \
-    else launch_pass<T, 1024, nmax_big<T>()>(KERN<T, 1024, nmax_big<T>()>, nblocks, lds, args, st);     \
+    else if ((n) <= 5120) launch_pass<T, 512, 5120>(KERN<T, 512, 5120>, nblocks, lds, args, st);      \
+    else if ((n) <= 10240) launch_pass<T, 1024, 10240>(KERN<T, 1024, 10240>, nblocks, lds, args, st); \
+    else launch_pass<T, 1024, nmax_big<T>()>(KERN<T, 1024, nmax_big<T>()>, nblocks, lds, args, st);    \
   } while (0)
 
 template <typename T>

@@ -61,10 +61,13 @@ class RingPlan {
   DftSet<double> dft_;                                       // one DFT description per distinct ring length
   DevBuf lens_;                                              // RingLen[nlengths]
   DevBuf lenidx_;                                            // int[nring]
-  DevBuf rings_[kDftMethods];                                // ring ids per DFT method
-  int nrings_m_[kDftMethods] = {0, 0, 0, 0};
-  int uniform_[kDftMethods] = {-1, -1, -1, -1};              // the one length index of a method's rings, or -2
-  size_t lds_[kDftMethods] = {0, 0, 0, 0};
+  // rings grouped by workgroup size, those with a split DFT apart (one launch each): ids, count, the one length index
+  // of the group's rings (or -2) and the LDS bytes of its longest
+  static constexpr int kRingGroups = 4;
+  DevBuf rings_[kRingGroups];
+  int nrings_m_[kRingGroups] = {};
+  int uniform_[kRingGroups];
+  size_t lds_[kRingGroups] = {};
   DevBuf theta_, phi0_, ofs_, weight_;
   DevBuf sqll_;  // sqrt(l(l+1))
   DevBuf G_;     // [nrows][nring] complex (m-major)
