@@ -333,8 +333,8 @@ template <typename T>
 struct InterpArgs {
   int nf, w, row_lo, nrow, spin, tr, tc, ntc, ntiles;
   T beta;
-  const T* kpoly;  // [(deg + 1)][w] kernel polynomials, one per footprint cell
-  int deg;
+  const T* kpoly;  // [(deg + 1)][w] kernel polynomials, one per footprint cell, and a row of zeros
+  int deg, deg_in;  // their degree: of the outer cells, of the others
   long npts;
   const double2* pts;
   const int* idx;
@@ -352,20 +352,76 @@ struct InterpArgs {
 // algebraically; there psi is below e^{-beta} * beta (~1e-8 at eps 1e-7) and the plan's fit still meets
 // max(eps/100, 1e-15) with the same degree as the interior cells (checked at plan time on 513 samples
 // per cell), so no exp / sqrt is evaluated per point.
+// FP64: psi is even and the fit mirrors it, c[k][W - 1 - i] = (-1)^k c[k][i], so cells i and W - 1 - i share the sums of
+// the even and of the odd powers: p_i = E + u O, p_{W-1-i} = E - u O, E and O Horner sums in u^2 (5 / 8 of the
+// multiply-adds of a sum per cell at degree 8); the powers above deg_in belong to the outer cells alone (eps 1e-10,
+// w = 11: 24 against 13).  FP32 keeps a sum per cell: the two forms differ by FP32 rounding, more in narrow kernels
+// (outer cells of degree 24 with large coefficients: 1e-4 at w = 2, 2e-6 at w = 4), and the spreading, which sums per
+// cell, has to stay the transpose.
+// The coefficients are read through the constant address space: wave-uniform scalar loads, which the compiler does not
+// choose by itself in a loop that also stores to global memory.
+template <typename T>
+using const_as = const __attribute__((address_space(4))) T;
+
 template <typename T, int W>
-__device__ __forceinline__ void ker_weights(double ft, double fp, T beta, const T* __restrict__ cp, int deg,
+__device__ __forceinline__ void ker_weights(double ft, double fp, const T* __restrict__ coef, int deg, int deg_in,
                                             T (&kt)[W], T (&kp)[W]) {
-  (void)beta;
+  const_as<T>* cp = (const_as<T>*)coef;
   const T ut = (T)(ft + 0.5 * W - 0.5), up = (T)(fp + 0.5 * W - 0.5);
-  const T* c = cp + (long)deg * W;
+  if constexpr (std::is_same<T, float>::value) {
+    const_as<T>* c = cp + (long)deg * W;
 #pragma unroll
-  for (int i = 0; i < W; ++i) { kt[i] = c[i]; kp[i] = c[i]; }
-  for (int k = deg - 1; k >= 0; --k) {
-    c -= W;
+    for (int i = 0; i < W; ++i) { kt[i] = c[i]; kp[i] = c[i]; }
+    for (int k = deg - 1; k >= 0; --k) {
+      c -= W;
 #pragma unroll
-    for (int i = 0; i < W; ++i) {
-      kt[i] = fma(kt[i], ut, c[i]);
-      kp[i] = fma(kp[i], up, c[i]);
+      for (int i = 0; i < W; ++i) {
+        kt[i] = fma(kt[i], ut, c[i]);
+        kp[i] = fma(kp[i], up, c[i]);
+      }
+    }
+  } else {
+    constexpr int H = W / 2;
+    const T vt = ut * ut, vp = up * up;
+    // kt[i], kp[i] hold E of cell i for i < H (and the middle cell) and O of cell W - 1 - i above
+    int k = deg & ~1;
+    const int kin = deg_in & ~1;
+    const_as<T>* c = cp + (long)k * W;
+    kt[0] = kp[0] = c[0];
+    kt[W - 1] = kp[W - 1] = c[W];
+    auto outer = [&] {
+      k -= 2;
+      c -= 2 * W;
+      kt[0] = fma(kt[0], vt, c[0]);
+      kp[0] = fma(kp[0], vp, c[0]);
+      kt[W - 1] = fma(kt[W - 1], vt, c[W]);
+      kp[W - 1] = fma(kp[W - 1], vp, c[W]);
+    };
+    while (k > kin) outer();
+#pragma unroll
+    for (int i = 1; i < W - H; ++i) kt[i] = kp[i] = c[i];
+#pragma unroll
+    for (int i = 1; i < H; ++i) kt[W - 1 - i] = kp[W - 1 - i] = c[W + i];
+    while (k > 0) {
+      outer();
+#pragma unroll
+      for (int i = 1; i < W - H; ++i) {
+        kt[i] = fma(kt[i], vt, c[i]);
+        kp[i] = fma(kp[i], vp, c[i]);
+      }
+#pragma unroll
+      for (int i = 1; i < H; ++i) {
+        kt[W - 1 - i] = fma(kt[W - 1 - i], vt, c[W + i]);
+        kp[W - 1 - i] = fma(kp[W - 1 - i], vp, c[W + i]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < H; ++i) {
+      const T et = kt[i], ot = kt[W - 1 - i], ep = kp[i], op = kp[W - 1 - i];
+      kt[i] = fma(ut, ot, et);
+      kt[W - 1 - i] = fma(-ut, ot, et);
+      kp[i] = fma(up, op, ep);
+      kp[W - 1 - i] = fma(-up, op, ep);
     }
   }
 }
@@ -382,8 +438,9 @@ __device__ __forceinline__ void interp_mark_bad(const InterpArgs<T>& a) {
   }
 }
 
-// Points per tile that the interpolation orders by bank class in LDS (tiles with more keep the binned order).
-constexpr int kInterpSortCap = 1024;
+// Points per tile that the interpolation orders by bank class in LDS (tiles with more keep the binned order): 4 KiB of
+// 16-bit entries, and full maps on ragged grids reach 1200 points per tile near the equator.
+constexpr int kInterpSortCap = 2048;
 
 // One workgroup per fine-grid tile: the tile plus its (W-1)-cell halo is staged in LDS once and
 // every point binned to the tile is interpolated from it (fully unrolled W x W footprint).
@@ -393,6 +450,14 @@ constexpr int kInterpSortCap = 1024;
 // its points per class base mod 16 (LDS atomics), lists them class by class, and gives lane position k the
 // list entry (k mod 16) S + k / 16, S = ceil(n / 16): the 16 lanes of a pass take entries S apart, from
 // (nearly always) different classes.
+// What bounds it: FP64 VALU issue, busy 67 % of the time at lmax 4095, about 870 instructions per point (the contraction
+// 266, its two weight vectors 100, the rotation 150, tile load and ordering 290), with the LDS reads beside it (144 of
+// 16 bytes at w = 12) and four workgroups per CU by their LDS.  With a Horner sum per cell in vector-loaded
+// coefficients, angles scaled and wrapped (a division) at every use, divisions in the tile load and at most 1024 ordered
+// points, and now: lmax 4095 spin 2 (w = 12, 33.5M points) 1.91 -> 1.29 ms, lmax 3001 (w = 11, 18M points) 1.68 -> 0.63,
+// HEALPix nside 512 at lmax 1000 (up to 1200 points per tile) 309 -> 121 us, lmax 255 23.6 -> 14.6 us, 20 000 points at
+// lmax 1024 58 -> 44 us, FP32 lmax 2047 (w = 9, 8.4M points) 291 -> 255 us.  Loading the tile row by row (uniform row
+// addresses) instead of cell by cell was 3 to 5 % slower.
 template <typename T, int W>
 __global__ __launch_bounds__(256) void k_interp_w(InterpArgs<T> a) {
   using T2 = c2_t<T>;
@@ -407,27 +472,46 @@ __global__ __launch_bounds__(256) void k_interp_w(InterpArgs<T> a) {
   if (s0 == s1) return;
   const int tw = a.tc + W, th = a.tr + W;
   int* ccnt = reinterpret_cast<int*>(smem_raw + sizeof(T2) * (size_t)tw * th);  // [16] class counts, then starts
-  int* order = ccnt + 16;                                                          // [kInterpSortCap]
+  unsigned short* order = reinterpret_cast<unsigned short*>(ccnt + 16);            // [kInterpSortCap]
   const int n = s1 - s0;
   const bool sorted = n <= kInterpSortCap;
   if (sorted && threadIdx.x < 16) ccnt[threadIdx.x] = 0;
   const int tile_r = tb / a.ntc, tile_c = tb - (tb / a.ntc) * a.ntc;
   const int r0 = tile_r * a.tr, c0 = tile_c * a.tc;
-  for (int i = threadIdx.x; i < tw * th; i += blockDim.x) {
-    const int rr = i / tw, cc = i - rr * tw;
-    const int grow = r0 + rr;
-    int gc = c0 + cc;
-    while (gc >= a.nf) gc -= a.nf;
-    tile[i] = grow < a.nrow ? a.grid[(long)grow * a.nf + gc] : T2{T(0), T(0)};
+  {
+    // cells i = thread + 256 e, four loads in flight; row and column advance without divisions, and cells past the
+    // tile or the formed rows load a clamped address
+    const int dr = 256 / tw, dc = 256 - dr * tw;
+    int rr = threadIdx.x / tw, cc = threadIdx.x - rr * tw;
+    for (int i = threadIdx.x; i < tw * th; i += 4 * 256) {
+      T2 v[4];
+      bool in[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int grow = r0 + rr;
+        int gc = c0 + cc;
+        gc -= gc >= a.nf ? a.nf : 0;
+        if (tw > a.nf) gc %= a.nf;  // a tile wider than a small grid
+        in[e] = grow < a.nrow;
+        v[e] = a.grid[(long)min(grow, a.nrow - 1) * a.nf + gc];
+        rr += dr;
+        cc += dc;
+        if (cc >= tw) {
+          cc -= tw;
+          ++rr;
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (i + e * 256 < tw * th) tile[i + e * 256] = in[e] ? v[e] : T2{T(0), T(0)};
+    }
   }
   __syncthreads();
-  const double scale = a.nf / (2.0 * M_PI);
   const double hw = 0.5 * W;
   // first cell of a point's footprint relative to the tile
   auto first_cell = [&](double2 tp, double& ut, double& up, int& i0, int& j0u, int& lr, int& lc) {
-    ut = tp.x * scale;
-    up = tp.y * scale;
-    up -= a.nf * floor(up / a.nf);
+    ut = tp.x;
+    up = tp.y;
     i0 = (int)ceil(ut - hw);
     j0u = (int)ceil(up - hw);
     const int j0 = j0u < 0 ? j0u + a.nf : j0u;
@@ -435,18 +519,21 @@ __global__ __launch_bounds__(256) void k_interp_w(InterpArgs<T> a) {
     lc = j0 - c0;
   };
   if (sorted) {
-    constexpr int EI = kInterpSortCap / 256;
+    constexpr int EI = kInterpSortCap / 256, EB = 4;
     int cls[EI], rank[EI];
 #pragma unroll
-    for (int e = 0; e < EI; ++e) {
-      const int i = threadIdx.x + e * 256;
-      cls[e] = rank[e] = 0;
-      if (i < n) {
+    for (int e = 0; e < EI; e += EB) {
+      if (e * 256 >= n) break;
+      double2 tp[EB];
+#pragma unroll
+      for (int b = 0; b < EB; ++b) tp[b] = a.pts[s0 + min((int)threadIdx.x + (e + b) * 256, n - 1)];
+#pragma unroll
+      for (int b = 0; b < EB; ++b) {
         double ut, up;
         int i0, j0u, lr, lc;
-        first_cell(a.pts[s0 + i], ut, up, i0, j0u, lr, lc);
-        cls[e] = (lr * tw + lc) & 15;
-        rank[e] = atomicAdd(&ccnt[cls[e]], 1);
+        first_cell(tp[b], ut, up, i0, j0u, lr, lc);
+        cls[e + b] = (lr * tw + lc) & 15;
+        if ((int)threadIdx.x + (e + b) * 256 < n) rank[e + b] = atomicAdd(&ccnt[cls[e + b]], 1);
       }
     }
     __syncthreads();
@@ -462,7 +549,7 @@ __global__ __launch_bounds__(256) void k_interp_w(InterpArgs<T> a) {
 #pragma unroll
     for (int e = 0; e < EI; ++e) {
       const int i = threadIdx.x + e * 256;
-      if (i < n) order[ccnt[cls[e]] + rank[e]] = i;
+      if (i < n) order[ccnt[cls[e]] + rank[e]] = (unsigned short)i;
     }
     __syncthreads();
   }
@@ -482,7 +569,7 @@ __global__ __launch_bounds__(256) void k_interp_w(InterpArgs<T> a) {
     const int o = a.idx[p];
     const bool ok = lr >= 0 && lr < a.tr && lc >= 0 && lc < a.tc;  // always true for binned points
     T kt[W], kp[W];
-    ker_weights<T, W>(i0 - ut, j0u - up, a.beta, a.kpoly, a.deg, kt, kp);
+    ker_weights<T, W>(i0 - ut, j0u - up, a.kpoly, a.deg, a.deg_in, kt, kp);
     T sr = 0, si = 0;
     if (ok) {
       const T2* base = tile + lr * tw + lc;
@@ -542,14 +629,11 @@ __global__ __launch_bounds__(256) void k_interp(InterpArgs<T> a) {
     tile[i] = grow < a.nrow ? a.grid[(long)grow * a.nf + gc] : T2{T(0), T(0)};
   }
   __syncthreads();
-  const double scale = a.nf / (2.0 * M_PI);
   const double hw = 0.5 * a.w;
   const T inv = (T)(2.0 / a.w);
   for (int p = s0 + threadIdx.x; p < s1; p += blockDim.x) {
     const double2 tp = a.pts[p];
-    const double ut = tp.x * scale;
-    double up = tp.y * scale;
-    up -= a.nf * floor(up / a.nf);
+    const double ut = tp.x, up = tp.y;
     const int i0 = (int)ceil(ut - hw);
     const int j0u = (int)ceil(up - hw);
     const int j0 = j0u < 0 ? j0u + a.nf : j0u;
@@ -659,7 +743,6 @@ __global__ __launch_bounds__(256) void k_spread_w(SpreadArgs<T> a) {
   __syncthreads();
   const int tile_r = tb / a.ntc, tile_c = tb % a.ntc;
   const int r0 = tile_r * a.tr, c0 = tile_c * a.tc;
-  const double scale = a.nf / (2.0 * M_PI);
   const double hw = 0.5 * W;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int row16 = lane >> 4;  // this lane's 16-lane row of the wave
@@ -675,9 +758,7 @@ __global__ __launch_bounds__(256) void k_spread_w(SpreadArgs<T> a) {
     T ut_ = T(0), up_ = T(0);
     if (p < s1) {
       const double2 tp = a.pts[p];
-      const double ut = tp.x * scale;
-      double up = tp.y * scale;
-      up -= a.nf * floor(up / a.nf);
+      const double ut = tp.x, up = tp.y;
       const int i0 = (int)ceil(ut - hw);
       const int j0u = (int)ceil(up - hw);
       const int j0 = j0u < 0 ? j0u + a.nf : j0u;
@@ -865,7 +946,6 @@ __global__ __launch_bounds__(256) void k_spread_rows(SpreadArgs<T> a, RowsLayout
   // segment's first row
   const int excl_c1 = a.ntc >= 2 ? min(a.tc, a.nf - c0) : 0;
   const int excl_r0 = t0 == 0 ? 0 : t0 * tr + W - 1, excl_r1 = t1 * tr;
-  const double scale = a.nf / (2.0 * M_PI);
   const double hw = 0.5 * W;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int l16 = lane & 15, gsub = lane >> 4;
@@ -879,9 +959,8 @@ __global__ __launch_bounds__(256) void k_spread_rows(SpreadArgs<T> a, RowsLayout
   // first cells of a binned point, relative to the tile; lr / lc outside the tile never happen
   auto cells = [&](int p, int r0, int& lr, int& lc, double& ut, double& up, int& i0, int& j0u) {
     const double2 tp = a.pts[p];
-    ut = tp.x * scale;
-    up = tp.y * scale;
-    up -= a.nf * floor(up / a.nf);
+    ut = tp.x;
+    up = tp.y;
     i0 = (int)ceil(ut - hw);
     j0u = (int)ceil(up - hw);
     const int j0 = j0u < 0 ? j0u + a.nf : j0u;
@@ -1144,7 +1223,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DM <= 12 ? 
   // cells no other workgroup touches, as in k_spread_rows
   const int excl_c1 = a.ntc >= 2 ? min(a.tc, a.nf - c0) : 0;
   const int excl_r0 = t0 == 0 ? 0 : t0 * tr + W - 1, excl_r1 = t1 * tr;
-  const double scale = a.nf / (2.0 * M_PI);
   const double hw = 0.5 * W;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int l16 = lane & 15, q16 = lane >> 4;
@@ -1153,9 +1231,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DM <= 12 ? 
   for (int k = 0; k <= DM; ++k) cf[k] = (l16 < W && k <= lay.deg) ? a.kpoly[(long)k * W + l16] : T(0);
   auto cells = [&](int p, int r0, int& lr, int& lc, double& ut, double& up, int& i0, int& j0u) {
     const double2 tp = a.pts[p];
-    ut = tp.x * scale;
-    up = tp.y * scale;
-    up -= a.nf * floor(up / a.nf);
+    ut = tp.x;
+    up = tp.y;
     i0 = (int)ceil(ut - hw);
     j0u = (int)ceil(up - hw);
     const int j0 = j0u < 0 ? j0u + a.nf : j0u;
@@ -1349,14 +1426,11 @@ __global__ __launch_bounds__(256) void k_spread(SpreadArgs<T> a) {
   __syncthreads();
   const int tile_r = tb / a.ntc, tile_c = tb % a.ntc;
   const int r0 = tile_r * a.tr, c0 = tile_c * a.tc;
-  const double scale = a.nf / (2.0 * M_PI);
   const double hw = 0.5 * a.w;
   const T inv = (T)(2.0 / a.w);
   for (int p = s0 + threadIdx.x; p < s1; p += blockDim.x) {
     const double2 tp = a.pts[p];
-    const double ut = tp.x * scale;
-    double up = tp.y * scale;
-    up -= a.nf * floor(up / a.nf);
+    const double ut = tp.x, up = tp.y;
     const int i0 = (int)ceil(ut - hw);
     const int j0u = (int)ceil(up - hw);
     const int j0 = j0u < 0 ? j0u + a.nf : j0u;
@@ -1437,6 +1511,9 @@ __device__ __forceinline__ RunInfo wave_runs(int key, bool valid) {
   return r;
 }
 
+// Position along phi in cells, in [0, nf] (nf for a tiny negative angle).
+__device__ __forceinline__ double wrap_cells(double up, int nf) { return fma(-(double)nf, floor(up / nf), up); }
+
 // Tile of a point, or a.ntiles (the bin after the last tile, which no interpolation or spreading tile reads)
 // for a point whose footprint leaves the formed rows or that is not finite.  The range checks come before
 // any float-to-int conversion, which is undefined for NaN and out-of-range values.
@@ -1444,15 +1521,14 @@ __device__ __forceinline__ int bin_key(const BinArgs& a, double theta, double ph
   const double scale = a.nf / (2.0 * M_PI);
   const double hw = 0.5 * a.w;
   const double ut = theta * scale;
-  double up = phi * scale;
+  const double up = phi * scale;
   const bool finite = ut > -4.0 * a.nf && ut < 4.0 * a.nf && fabs(phi) < 1e15;  // false for NaN
   if (!finite) {
     bad = true;
     return a.ntiles;
   }
-  up -= a.nf * floor(up / a.nf);
   const int q0 = (int)ceil(ut - hw) - a.row_lo;
-  int j0 = (int)ceil(up - hw);
+  int j0 = (int)ceil(wrap_cells(up, a.nf) - hw);
   if (j0 < 0) j0 += a.nf;
   if (j0 >= a.nf) j0 -= a.nf;
   bad = q0 < 0 || q0 + a.w > a.nrow;
@@ -1474,7 +1550,10 @@ __global__ __launch_bounds__(256) void k_bin_count(BinArgs a, int* bad_count) {
   if (valid && r.leader == (int)(threadIdx.x & 63)) atomicAdd(&a.cnt[k], r.len);
 }
 
-__global__ __launch_bounds__(256) void k_bin_scatter(long npts, const double* __restrict__ theta,
+// Points in tile order, as positions in cells of the fine grid along both axes: every pass over them (one per map for
+// maps that share a deflection, two of the interpolation) starts from these, without the angles' scaling, wrapping and
+// its division.
+__global__ __launch_bounds__(256) void k_bin_scatter(long npts, int nf, const double* __restrict__ theta,
                                                      const double* __restrict__ phi, const int* __restrict__ key,
                                                      const int* __restrict__ start, int* cursor,
                                                      double2* __restrict__ pts, int* __restrict__ idx) {
@@ -1488,7 +1567,8 @@ __global__ __launch_bounds__(256) void k_bin_scatter(long npts, const double* __
   base = __shfl(base, r.leader, 64);
   if (!valid) return;
   const int pos = base + (lane - r.leader);
-  pts[pos] = double2{theta[j], phi[j]};
+  const double scale = nf / (2.0 * M_PI);
+  pts[pos] = double2{theta[j] * scale, wrap_cells(phi[j] * scale, nf)};
   idx[pos] = (int)j;
 }
 
@@ -1641,23 +1721,31 @@ NufftParams NufftParams::choose(int lmax, int spin, double eps, double sigma_hin
 // outer cells hold the square-root branch point at |z| = 1, where psi is already below
 // e^{-beta (1 - sqrt(1 - (1 - 2/w)^2))} ~ eps, so their fit error stays below the target as well.
 // The degree is the lowest in [2, 24] whose max error on a dense sample (evaluated by Horner in
-// the working precision) over all cells is below `target`.
-static void fit_kernel_poly(int w, double beta, double target, bool single, int& deg, double& err,
+// the working precision) over all cells is below `target` (24 if none is).  The outer cells set it: when
+// the interior cells reach a hundredth of their error (or the rounding) at a lower degree, those are fitted again
+// at that degree, odd, and hold zeros above it (deg_in; deg otherwise).
+static void fit_kernel_poly(int w, double beta, double target, bool single, int& deg, int& deg_in, double& err,
                             std::vector<double>& coef) {
   const int ni = w;  // every cell of the footprint, the two outer ones included (see ker_weights)
-  deg = 0; err = 0; coef.clear();
+  deg = deg_in = 0; err = 0; coef.clear();
   if (ni <= 0) return;
   auto psi = [&](long double z) -> long double {
     long double t = 1.0L - z * z;
     return t > 0 ? std::exp((long double)beta * (std::sqrt(t) - 1.0L)) : 0.0L;
   };
-  double best_err = 1e300;
-  for (int d = 2; d <= 24; ++d) {
+  constexpr int NQ = 513;  // samples per cell
+  std::vector<long double> ref((size_t)ni * NQ);
+  for (int i = 0; i < ni; ++i)
+    for (int q = 0; q < NQ; ++q) {
+      const double u = -0.5 + q / (NQ - 1.0);
+      ref[(size_t)i * NQ + q] = psi((u + 0.5L + i - 0.5L * w) * 2.0L / w);
+    }
+  // fits cells i0 .. ni - 1 - i0 at degree d (FP64: the first half, the others by mirroring)
+  auto fit = [&](int d, int i0, std::vector<double>& c) {
     const int n = d + 1;
-    std::vector<double> c((size_t)n * ni);
     std::vector<long double> un(n);
     for (int j = 0; j < n; ++j) un[j] = 0.5L * std::cos((long double)M_PI * (j + 0.5L) / n);
-    for (int i = 0; i < ni; ++i) {
+    for (int i = i0; i < (single ? ni - i0 : (ni + 1) / 2); ++i) {
       // Vandermonde solve in long double (Gaussian elimination, partial pivoting)
       std::vector<long double> A((size_t)n * (n + 1));
       for (int r = 0; r < n; ++r) {
@@ -1682,12 +1770,21 @@ static void fit_kernel_poly(int w, double beta, double target, bool single, int&
         for (int k = r + 1; k < n; ++k) v -= A[(size_t)r * (n + 1) + k] * x[k];
         x[r] = v / A[(size_t)r * (n + 1) + r];
       }
-      for (int k = 0; k < n; ++k) c[(size_t)k * ni + i] = (double)x[k];
+      // psi is even: the mirrored cell has the same polynomial in -u, the middle cell no odd powers
+      const int im = single ? i : ni - 1 - i;
+      for (size_t k = 0; k * ni < c.size(); ++k) {
+        const double xk = (int)k > d || (!single && i == im && k % 2) ? 0.0 : (double)x[k];
+        c[k * ni + im] = k % 2 ? -xk : xk;
+        c[k * ni + i] = xk;
+      }
     }
+  };
+  // max error of cells i0 .. ni - 1 - i0 at degree d
+  auto error = [&](int d, int i0, const std::vector<double>& c) {
     double e = 0;
-    for (int i = 0; i < ni; ++i)
-      for (int q = 0; q <= 512; ++q) {
-        const double u = -0.5 + q / 512.0;
+    for (int i = i0; i < ni - i0; ++i)
+      for (int q = 0; q < NQ; ++q) {
+        const double u = -0.5 + q / (NQ - 1.0);
         double v;
         if (single) {
           float fv = (float)c[(size_t)d * ni + i];
@@ -1697,12 +1794,31 @@ static void fit_kernel_poly(int w, double beta, double target, bool single, int&
           v = c[(size_t)d * ni + i];
           for (int k = d - 1; k >= 0; --k) v = std::fma(v, u, c[(size_t)k * ni + i]);
         }
-        e = std::max(e, (double)std::fabs((long double)v - psi((u + 0.5L + i - 0.5L * w) * 2.0L / w)));
+        e = std::max(e, (double)std::fabs((long double)v - ref[(size_t)i * NQ + q]));
       }
+    return e;
+  };
+  double best_err = 1e300;
+  for (int d = 2; d <= 24; ++d) {
+    std::vector<double> c((size_t)(d + 1) * ni);
+    fit(d, 0, c);
+    const double e = error(d, 0, c);
     if (e < best_err) { best_err = e; deg = d; coef = c; }
     if (e <= target) break;
   }
   err = best_err;
+  deg_in = deg;
+  if (single) return;
+  const double in_target = std::max(best_err / 100.0, 5e-16);
+  for (int d = 5; d + 2 <= deg; d += 2) {
+    std::vector<double> c = coef;
+    fit(d, 1, c);
+    if (error(d, 1, c) <= in_target) {
+      coef = c;
+      deg_in = d;
+      return;
+    }
+  }
 }
 
 NufftPlan::NufftPlan(const NufftParams& p, long npts_max, hipStream_t st, int tile_rows)
@@ -1726,9 +1842,9 @@ NufftPlan::NufftPlan(const NufftParams& p, long npts_max, hipStream_t st, int ti
   {
     std::vector<double> c;
     const double target = std::max(p.eps / 100.0, p.single ? 3e-7 : 1e-15);
-    fit_kernel_poly(p.w, p.beta, target, p.single, p_.poly_deg, p_.poly_err, c);
+    fit_kernel_poly(p.w, p.beta, target, p.single, p_.poly_deg, p_.poly_deg_in, p_.poly_err, c);
     fitted = !c.empty();
-    if (c.empty()) c.push_back(0.0);
+    c.resize(c.size() + p.w, 0.0);  // the sums of odd powers start one row up when the degree is even
     if (p.single) {
       std::vector<float> cf(c.begin(), c.end());
       upload(kpoly_, cf);
@@ -1820,7 +1936,7 @@ void NufftPlan::set_pts(const double* theta, const double* phi, long npts, hipSt
   size_t tb = scan_tmp_bytes_;
   NUSHT_HIP(hipcub::DeviceScan::ExclusiveSum(scan_tmp_.get(), tb, tile_cnt_.as<int>(), tile_start_.as<int>(),
                                              ntiles + 1, st));
-  hipLaunchKernelGGL(k_bin_scatter, dim3(ceil_div(npts, 256)), dim3(256), 0, st, npts, theta, phi, key_.as<int>(),
+  hipLaunchKernelGGL(k_bin_scatter, dim3(ceil_div(npts, 256)), dim3(256), 0, st, npts, p_.nf, theta, phi, key_.as<int>(),
                      tile_start_.as<int>(), cursor_.as<int>(), pts_.as<double2>(), idx_.as<int>());
   NUSHT_LAUNCH_CHECK();
   if (!check) return;
@@ -1882,11 +1998,11 @@ void NufftPlan::type2_impl(const double2* G, long sm, const double* gamma, doubl
   if (npts_ == 0) return;
   const int ntiles = ntile_r_ * ntile_c_;
   InterpArgs<T> ia{p.nf, p.w, p.row_lo, p.nrow, p.spin, tile_r_, tile_c_, ntile_c_, ntiles, (T)p.beta,
-                   kpoly_.as<T>(), p.poly_deg, npts_, pts_.as<double2>(), idx_.as<int>(), tile_start_.as<int>(),
+                   kpoly_.as<T>(), p.poly_deg, p.poly_deg_in, npts_, pts_.as<double2>(), idx_.as<int>(), tile_start_.as<int>(),
                    grid_.as<T2>(), gamma, ore, oim};
   StageScope sc("nufft_interp", st);
   // tile, then (templated widths) the class counts and the point order
-  const size_t tlds = sizeof(T2) * (size_t)(tile_r_ + p.w) * (tile_c_ + p.w) + sizeof(int) * (16 + kInterpSortCap);
+  const size_t tlds = sizeof(T2) * (size_t)(tile_r_ + p.w) * (tile_c_ + p.w) + sizeof(int) * 16 + sizeof(unsigned short) * kInterpSortCap;
   launch_interp<T, 2>(p.w, dim3(ntiles + 1), tlds, st, ia);  // + 1: the workgroup for out-of-range points
   NUSHT_LAUNCH_CHECK();
 }
