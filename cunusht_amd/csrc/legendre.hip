@@ -1504,6 +1504,11 @@ static void legendre_synth_chunk(const LegendreTables& t, int nmaps, int ncomp, 
 
 int legendre_variant_count() { return kNumSynVariants; }
 
+// Waves of a one-group launch (m times ring groups) below which a table takes the row-broadcast synthesis unmeasured.
+// At lmax 255 (768 waves, spin 0) it takes 10 us against 22, at lmax 1000 (8008) 0.070 to 0.160 ms against 0.118 to
+// 0.218; between 20 us launches the measurement took the slower one in one process of four.
+constexpr long kRowWaves = 4096;
+
 void legendre_autotune(LegendreTables& t, int ncomp, double2* coef_ws, double2* G, long sm, long sr, hipStream_t st) {
   // NUSHT_LEGENDRE_VARIANT=k fixes the variant (tests run every variant this way)
   if (const char* fv = getenv("NUSHT_LEGENDRE_VARIANT"); fv && fv[0]) {
@@ -1515,6 +1520,11 @@ void legendre_autotune(LegendreTables& t, int ncomp, double2* coef_ws, double2* 
   }
   const bool gr = t.spin > 0 && ncomp == 1;
   int& slot = gr ? t.variant_grad : t.variant;
+  // Few waves: the row broadcasts are up to twice as fast, while launches this short are not told apart by their times
+  if ((long)(t.lmax + 1) * t.ngroups < kRowWaves) {
+    slot = 0;
+    return;
+  }
   // one measurement per (lmax, spin, ring pairs) and process
   static std::mutex mu;
   static std::map<std::tuple<int, int, int, int>, std::pair<int, float>> cache;
