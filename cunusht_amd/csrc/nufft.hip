@@ -1967,9 +1967,12 @@ static constexpr int nmax_big() { return kLdsBytes / (int)sizeof(c2_t<T>); }
 // workgroups; several cover each other's barriers, loads and stores.
 // With 1024 threads for every length above 2048 and now, theta and phi pass: lmax 1024 FP64 (grid near 2560) 74 -> 56
 // and 70 -> 48 us, lmax 2047 FP32 (5120) 152 -> 81 and 180 -> 70 us.
+// 256 threads up to 2560, where four workgroups' rows just fill the LDS, instead of up to 2048: HEALPix lmax 1000 (2560)
+// 55 -> 42 and 39 -> 33 us; 320 threads up to 3200 were slower than 512 (lmax 1024, grid 2592: 61 and 56 us).
 #define NUSHT_LAUNCH_SIZED(KERN, T, n, nblocks, lds, args, st)                                        \
   do {                                                                                               \
     if ((n) <= 2048) launch_pass<T, 256, 2048>(KERN<T, 256, 2048>, nblocks, lds, args, st);           \
+    else if ((n) <= 2560) launch_pass<T, 256, 2560>(KERN<T, 256, 2560>, nblocks, lds, args, st);      \
     else if ((n) <= 5120) launch_pass<T, 512, 5120>(KERN<T, 512, 5120>, nblocks, lds, args, st);      \
     else if ((n) <= 10240) launch_pass<T, 1024, 10240>(KERN<T, 1024, 10240>, nblocks, lds, args, st); \
     else launch_pass<T, 1024, nmax_big<T>()>(KERN<T, 1024, nmax_big<T>()>, nblocks, lds, args, st);    \
@@ -2002,7 +2005,8 @@ void NufftPlan::type2_impl(const double2* G, long sm, const double* gamma, doubl
                    grid_.as<T2>(), gamma, ore, oim};
   StageScope sc("nufft_interp", st);
   // tile, then (templated widths) the class counts and the point order
-  const size_t tlds = sizeof(T2) * (size_t)(tile_r_ + p.w) * (tile_c_ + p.w) + sizeof(int) * 16 + sizeof(unsigned short) * kInterpSortCap;
+  const size_t tlds = sizeof(T2) * (size_t)(tile_r_ + p.w) * (tile_c_ + p.w) + sizeof(int) * 16 +
+                      sizeof(unsigned short) * kInterpSortCap;
   launch_interp<T, 2>(p.w, dim3(ntiles + 1), tlds, st, ia);  // + 1: the workgroup for out-of-range points
   NUSHT_LAUNCH_CHECK();
 }
