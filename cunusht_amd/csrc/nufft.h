@@ -98,9 +98,8 @@ class NufftPlan {
   DevBuf pts_;                     // double2[npts_max] sorted points, positions in fine cells along theta and phi
   DevBuf idx_;                     // int[npts_max] original index of sorted point
   DevBuf tile_start_;              // int[ntiles + 1]
-  DevBuf tile_cnt_;                // int[ntiles + 1]
+  DevBuf tile_cnt_;                // int[ntiles + 1] counts, an error counter, int[ntiles + 1] scatter cursors
   DevBuf key_;                     // int[npts_max] tile of each point
-  DevBuf cursor_;                  // int[ntiles]
   DevBuf scan_tmp_;                // hipcub scan temp storage
   size_t scan_tmp_bytes_ = 0;
 };

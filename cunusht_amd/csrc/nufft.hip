@@ -1901,8 +1901,7 @@ NufftPlan::NufftPlan(const NufftParams& p, long npts_max, hipStream_t st, int ti
   idx_.alloc(sizeof(int) * npts_max_);
   key_.alloc(sizeof(int) * npts_max_);
   tile_start_.alloc(sizeof(int) * (ntiles + 1));
-  tile_cnt_.alloc(sizeof(int) * (ntiles + 2));
-  cursor_.alloc(sizeof(int) * (ntiles + 1));
+  tile_cnt_.alloc(sizeof(int) * (2 * (size_t)ntiles + 3));
   NUSHT_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, scan_tmp_bytes_, tile_cnt_.as<int>(), tile_start_.as<int>(),
                                              ntiles + 1, st));
   scan_tmp_.alloc(std::max<size_t>(scan_tmp_bytes_, 16));
@@ -1910,7 +1909,7 @@ NufftPlan::NufftPlan(const NufftParams& p, long npts_max, hipStream_t st, int ti
 
 size_t NufftPlan::bytes() const {
   return deconv_.bytes() + kpoly_.bytes() + T_.bytes() + grid_.bytes() + pts_.bytes() + idx_.bytes() + key_.bytes() +
-         tile_start_.bytes() + tile_cnt_.bytes() + cursor_.bytes() + scan_tmp_.bytes();
+         tile_start_.bytes() + tile_cnt_.bytes() + scan_tmp_.bytes();
 }
 
 void NufftPlan::set_pts(const double* theta, const double* phi, long npts, hipStream_t st, bool check) {
@@ -1918,11 +1917,11 @@ void NufftPlan::set_pts(const double* theta, const double* phi, long npts, hipSt
   npts_ = npts;
   StageScope sc("set_pts", st);
   const int ntiles = ntile_r_ * ntile_c_;
-  // tile_cnt_[ntiles + 1] is an error counter
-  hipLaunchKernelGGL(k_fill_zero<int>, dim3(ceil_div(ntiles + 2, 256)), dim3(256), 0, st, tile_cnt_.as<int>(),
-                     (long)ntiles + 2);
-  hipLaunchKernelGGL(k_fill_zero<int>, dim3(ceil_div(ntiles + 1, 256)), dim3(256), 0, st, cursor_.as<int>(),
-                     (long)ntiles + 1);
+  // tile_cnt_[ntiles + 1] is an error counter; the scatter's cursors follow it, cleared by the same launch (2 to 4 us
+  // of a small plan's call)
+  int* cursor = tile_cnt_.as<int>() + ntiles + 2;
+  hipLaunchKernelGGL(k_fill_zero<int>, dim3(ceil_div(2 * (long)ntiles + 3, 256)), dim3(256), 0, st,
+                     tile_cnt_.as<int>(), 2 * (long)ntiles + 3);
   NUSHT_LAUNCH_CHECK();
   if (npts == 0) {
     hipLaunchKernelGGL(k_fill_zero<int>, dim3(ceil_div(ntiles + 1, 256)), dim3(256), 0, st, tile_start_.as<int>(),
@@ -1937,7 +1936,7 @@ void NufftPlan::set_pts(const double* theta, const double* phi, long npts, hipSt
   NUSHT_HIP(hipcub::DeviceScan::ExclusiveSum(scan_tmp_.get(), tb, tile_cnt_.as<int>(), tile_start_.as<int>(),
                                              ntiles + 1, st));
   hipLaunchKernelGGL(k_bin_scatter, dim3(ceil_div(npts, 256)), dim3(256), 0, st, npts, p_.nf, theta, phi, key_.as<int>(),
-                     tile_start_.as<int>(), cursor_.as<int>(), pts_.as<double2>(), idx_.as<int>());
+                     tile_start_.as<int>(), cursor, pts_.as<double2>(), idx_.as<int>());
   NUSHT_LAUNCH_CHECK();
   if (!check) return;
   int bad = 0;
