@@ -1721,9 +1721,10 @@ NufftParams NufftParams::choose(int lmax, int spin, double eps, double sigma_hin
 // outer cells hold the square-root branch point at |z| = 1, where psi is already below
 // e^{-beta (1 - sqrt(1 - (1 - 2/w)^2))} ~ eps, so their fit error stays below the target as well.
 // The degree is the lowest in [2, 24] whose max error on a dense sample (evaluated by Horner in
-// the working precision) over all cells is below `target` (24 if none is).  The outer cells set it: when
-// the interior cells reach a hundredth of their error (or the rounding) at a lower degree, those are fitted again
-// at that degree, odd, and hold zeros above it (deg_in; deg otherwise).
+// the working precision) over all cells is below `target` (24 if none is).  The outer cells set it: when the
+// interior cells are as exact at a lower degree, those are fitted again at that degree, odd, and hold zeros above it
+// (deg_in; deg otherwise).  As exact: their error is that of the fit at deg or half an ulp of the largest weight, 1.
+// Where deg is 24 that is degree 15 or 17 (errors 0.8 to 1.3e-16).
 static void fit_kernel_poly(int w, double beta, double target, bool single, int& deg, int& deg_in, double& err,
                             std::vector<double>& coef) {
   const int ni = w;  // every cell of the footprint, the two outer ones included (see ker_weights)
@@ -1809,7 +1810,7 @@ static void fit_kernel_poly(int w, double beta, double target, bool single, int&
   err = best_err;
   deg_in = deg;
   if (single) return;
-  const double in_target = std::max(best_err / 100.0, 5e-16);
+  const double in_target = std::max(error(deg, 1, coef), 0x1p-53);
   for (int d = 5; d + 2 <= deg; d += 2) {
     std::vector<double> c = coef;
     fit(d, 1, c);
