@@ -1570,11 +1570,19 @@ void legendre_autotune(LegendreTables& t, int ncomp, double2* coef_ws, double2* 
   cache[key] = {bestv, best / 2};
 }
 
-// Waves of a launch with three ring groups each from which the adjoint takes three groups per wave: below it a SIMD
-// has one or two waves, and the shorter l-step of one group is worth more than the shared lane sums.  Measured, ms, one /
-// three groups: lmax 700 spin 0 0.090 / 0.096, spin 2 0.167 / 0.174 (1402 waves); lmax 850 0.120 / 0.122, 0.224 / 0.231
-// (2553); lmax 1000 0.170 / 0.148, 0.296 / 0.276 (3003).
+// Ring groups per wave of the adjoint.  Up to 384 ring pairs (512 for spin 0) one or two waves hold an m: their sums on a
+// cleared output come out the same in either order, so the adjoint repeats bit for bit (with one group per wave, three or
+// more waves at lmax 300 / 511 / 766: spin 2 0.048 / 0.086 / 0.198 ms, now 0.054 / 0.108 / 0.198).  Above, three or more
+// waves add in any order, and the choice is by time: three groups once a launch with three has kAdjointMinWaves waves; below it a
+// SIMD has one or two waves, and the shorter l-step of one group is worth more than the shared lane sums.  Measured, ms,
+// one / three groups: lmax 700 spin 0 0.090 / 0.096, spin 2 0.167 / 0.174 (1402 waves); lmax 850 0.120 / 0.122,
+// 0.224 / 0.231 (2553); lmax 1000 0.170 / 0.148, 0.296 / 0.276 (3003).
 constexpr long kAdjointMinWaves = 2600;
+
+static int adjoint_groups(int mode, int lmax, int ngroups) {
+  if (ngroups <= (mode == kScalar ? 8 : 6)) return ceil_div(ngroups, 2);
+  return (long)(lmax + 1) * ceil_div(ngroups, 3) < kAdjointMinWaves ? 1 : 3;
+}
 
 template <int MODE>
 static void launch_adjoint(const LegendreTables& t, AdjArgs a, hipStream_t st) {
@@ -1582,10 +1590,12 @@ static void launch_adjoint(const LegendreTables& t, AdjArgs a, hipStream_t st) {
   const long n = (long)(L + 1) * (L + 2) / 2 * (MODE == kFull ? 2 : 1);
   hipLaunchKernelGGL(k_adjoint_clear, dim3((unsigned)std::min<long>(4096, (n + 255) / 256)), dim3(256), 0, st, a.alm, n);
   NUSHT_LAUNCH_CHECK();
-  const int R = (long)(L + 1) * ceil_div(t.ngroups, 3) < kAdjointMinWaves ? 1 : 3;
+  const int R = adjoint_groups(MODE, L, t.ngroups);
   a.nsb = ceil_div(t.ngroups, R) | 1;  // odd, as in launch_synth
   const dim3 grid((unsigned)(a.nsb * ceil_div(L + 1, kNumXcd) * kNumXcd));
   if (R == 1) hipLaunchKernelGGL((k_adjoint<MODE, 1>), grid, dim3(64), 0, st, a);
+  else if (R == 2) hipLaunchKernelGGL((k_adjoint<MODE, 2>), grid, dim3(64), 0, st, a);
+  else if (MODE == kScalar && R == 4) hipLaunchKernelGGL((k_adjoint<kScalar, 4>), grid, dim3(64), 0, st, a);
   else hipLaunchKernelGGL((k_adjoint<MODE, 3>), grid, dim3(64), 0, st, a);
   NUSHT_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_adjoint_finish<MODE>, dim3(ceil_div(L + 1, 1024), L / 2 + 1), dim3(256), 0, st, L, t.spin,

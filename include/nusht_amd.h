@@ -129,7 +129,9 @@ int nusht_ringplan_synthesis(nusht_ringplan_t p, const double* alm, int ncomp, d
  * CPU_sht_transformer.py:37-48 ducc adjoint_synthesis with apply_weights) */
 int nusht_ringplan_analysis(nusht_ringplan_t p, const double* map0, const double* map1, double* alm, int ncomp,
                             nusht_stream_t s);
-/* exact adjoint of the synthesis (no weights) */
+/* exact adjoint of the synthesis (no weights).  Repeats bit for bit up to 384 ring pairs (512 for spin 0: Gauss-Legendre
+ * grids of lmax 767 and 1023), as does nusht_ringplan_analysis; with more, FP64 sums meet in any order and results
+ * differ by rounding. */
 int nusht_ringplan_adjoint(nusht_ringplan_t p, const double* map0, const double* map1, double* alm, int ncomp,
                            nusht_stream_t s);
 /* spin-1 plans: gradient of a scalar field, (d/dtheta, d/dphi / sin theta) of f = sum alm Y_lm on the ring
