@@ -49,10 +49,10 @@ __device__ __forceinline__ void bluestein_lds(c2_t<T>* buf, int n, const DftLen<
   const int M = L.mlen;
   for (int j = threadIdx.x; j < M; j += NT) buf[j] = j < n ? cmul(buf[j], L.chirp[j]) : T2{T(0), T(0)};
   __syncthreads();
-  fft_lds<T, NT, NMAX, true>(buf, L.fd);
+  [[clang::always_inline]] fft_lds<T, NT, NMAX, true>(buf, L.fd);
   for (int j = threadIdx.x; j < M; j += NT) buf[j] = cconj(cmul(buf[j], L.kern[j]));
   __syncthreads();
-  fft_lds<T, NT, NMAX, true>(buf, L.fd);
+  [[clang::always_inline]] fft_lds<T, NT, NMAX, true>(buf, L.fd);
   const T inv = T(1) / T(M);
   for (int k = threadIdx.x; k < n; k += NT) buf[k] = cscale(cmul(L.chirp[k], cconj(buf[k])), inv);
   __syncthreads();
@@ -65,7 +65,7 @@ __device__ __forceinline__ void dft_lds(c2_t<T>* buf, const DftLen<T>& L) {
   const int n = L.n;
   constexpr int E = (NMAX + NT - 1) / NT;  // values per thread held in registers
   if constexpr (METHOD == (int)DftMethod::Direct) {
-    fft_lds<T, NT, NMAX, true>(buf, L.fd);
+    [[clang::always_inline]] fft_lds<T, NT, NMAX, true>(buf, L.fd);
     return;
   }
   if constexpr (METHOD == (int)DftMethod::Bluestein) {
@@ -93,7 +93,7 @@ __device__ __forceinline__ void dft_lds(c2_t<T>* buf, const DftLen<T>& L) {
       if (L.sub_bluestein) {
         bluestein_lds<T, NT, NMAX>(buf, b, L);
       } else {
-        fft_lds<T, NT, NMAX, true>(buf, L.fd);
+        [[clang::always_inline]] fft_lds<T, NT, NMAX, true>(buf, L.fd);
       }
 #pragma unroll
       for (int i = 0; i < E; ++i) {
@@ -137,7 +137,7 @@ __device__ __forceinline__ void dft_lds(c2_t<T>* buf, const DftLen<T>& L) {
     if (q < n1) buf[q] = v[i];
   }
   __syncthreads();
-  fft_lds<T, NT, NMAX, true>(buf, L.fd);
+  [[clang::always_inline]] fft_lds<T, NT, NMAX, true>(buf, L.fd);
   const T2 a0 = buf[0];
 #pragma unroll
   for (int i = 0; i < E; ++i) v[i] = L.kern[min((int)threadIdx.x + i * NT, n1 - 1)];
@@ -148,7 +148,7 @@ __device__ __forceinline__ void dft_lds(c2_t<T>* buf, const DftLen<T>& L) {
     if (q < n1) buf[q] = cconj(cmul(buf[q], v[i]));
   }
   __syncthreads();
-  fft_lds<T, NT, NMAX, true>(buf, L.fd);
+  [[clang::always_inline]] fft_lds<T, NT, NMAX, true>(buf, L.fd);
   const T inv = T(1) / T(n1);
 #pragma unroll
   for (int i = 0; i < E; ++i) {

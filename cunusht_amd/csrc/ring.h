@@ -61,13 +61,15 @@ class RingPlan {
   DftSet<double> dft_;                                       // one DFT description per distinct ring length
   DevBuf lens_;                                              // RingLen[nlengths]
   DevBuf lenidx_;                                            // int[nring]
-  // rings grouped by workgroup size, those with a split DFT apart (one launch each): ids, count, the one length index
-  // of the group's rings (or -2) and the LDS bytes of its longest
-  static constexpr int kRingGroups = 4;
-  DevBuf rings_[kRingGroups];
-  int nrings_m_[kRingGroups] = {};
-  int uniform_[kRingGroups];
-  size_t lds_[kRingGroups] = {};
+  // one launch over part of the rings: direction (RingPass), workgroup size, DFT method, length index shared by its rings
+  // (or -1), whether rows that alias are staged, number and ids of the rings, LDS bytes of the longest
+  struct RingGroup {
+    int pass, cls, method, one, stage, n;
+    size_t lds;
+    DevBuf ids;
+  };
+  std::vector<RingGroup> groups_;
+  void group_rings(const std::vector<int>& lidx, bool to_rings);
   DevBuf theta_, phi0_, ofs_, weight_;
   DevBuf sqll_;  // sqrt(l(l+1))
   DevBuf G_;     // [nrows][nring] complex (m-major)

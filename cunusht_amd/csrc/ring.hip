@@ -10,18 +10,29 @@
 
 #include <algorithm>
 #include <cmath>
+#include <map>
+#include <set>
+#include <utility>
 
 namespace nusht {
 namespace {
 
-// Workgroup sizes by the values a ring's DFT holds in LDS.  Every thread keeps about eight values in registers (105 -
-// 127 VGPRs, four waves per SIMD), so a workgroup of the largest size fills a CU whatever its ring's length; with
-// smaller ones four rings of up to 2048 values, or two of up to 4160, run on a CU and cover each other's barriers
-// and loads.  Measured with 768 threads for every ring and now: 301 rings of 625 values (lmax 300)
+// Workgroup sizes by the values a ring's DFT holds in LDS.  Every thread keeps about eight values in registers (106 -
+// 128 VGPRs, four waves per SIMD; three of the largest workgroup), so a workgroup of the largest size fills a CU whatever
+// its ring's length; with smaller ones four rings of up to 2048 values, or two of up to 4160, run on a CU and cover each
+// other's barriers and loads.  Measured with 768 threads for every ring and now: 301 rings of 625 values (lmax 300)
 // 28 -> 21 us; 1501 rings of 3072 values (lmax 1500), synthesis 100 -> 70 us, adjoint 94 -> 78 us.
+// Registers spilled at the small sizes: none or a few for direct and Bluestein transforms (13 to 30 where rings alias),
+// 30 to 112 for Rader's and for the launches of any method.
 constexpr int kRingClasses = 3;
 constexpr int kRingNT[kRingClasses] = {256, 512, kDftNT};
 constexpr int kRingNMax[kRingClasses] = {2048, 4160, kDftNMAX};
+
+// A plan of at most kFewRings rings, the longest above kFewRingsValues, runs as one launch of its longest ring's size and
+// at least 512 threads: at most two workgroups come to a CU, so a launch lasts as long as its slowest ring.  Adjoint /
+// synthesis, us, by each ring's size and now: 500 rings of 1001 to 2048 pixels 73 / 81 -> 48 / 53, 300 of 401 to 2000
+// 57 / 64 -> 36 / 39, 100 rings of 2000 15.3 / 16.0 -> 13.7 / 15.6.
+constexpr int kFewRings = 512, kFewRingsValues = 1024;
 
 // LDS values of a ring's workgroup: its DFT and, for a ring shorter than its band, the rows that alias onto it
 // (those of a band that does not fit are read term by term)
@@ -29,8 +40,7 @@ int ring_values(const RingLen& d, int nrow, int band) {
   return d.n >= band || nrow > kDftNMAX ? d.lds_values() : std::max(d.lds_values(), nrow);
 }
 
-int ring_class(const RingLen& d, int values) {
-  if (d.method == (int)DftMethod::Split) return kRingClasses - 1;  // long rings only
+int ring_class(int values) {
   int c = 0;
   while (values > kRingNMax[c]) ++c;
   return c;
@@ -66,12 +76,16 @@ __device__ __forceinline__ double2 ring_coef(const double2* g, int m, int L, int
   return v;
 }
 
-// UNIFORM: every ring of the launch has the length a.one >= 2 lmax + 1 (read from the kernel arguments) and the DFT method
-// METHOD; otherwise each ring reads its description from a.lens, may be shorter than its band and, with kAnyMethod,
-// takes its own method (all but the split): ragged grids run as one launch per workgroup size, since every launch
-// lasts as long as its slowest ring (HEALPix nside 512, lmax 1000: 218 us, 241 us with one launch per DFT method).
 constexpr int kAnyMethod = -1;
 
+// What a launch does: rows -> rings, every ring at least as long as its band; rows -> rings of any length; or the
+// transpose.  Each has a kernel of its own: the sums over aliased rows hold more registers than the rest.
+enum RingPass { kFullBand, kAliased, kToRows };
+
+// UNIFORM: every ring of the launch has the length a.one (read from the kernel arguments) and the DFT method METHOD;
+// otherwise each ring reads its description from a.lens and, with kAnyMethod, takes its own method (all but the split).
+// The transforms of every launch are inlined: called, they saved 160 to 250 bytes of registers per thread and shared
+// nothing with the loads around them (HEALPix nside 512, lmax 1000, spin 2: synthesis 166 -> 117 us, adjoint 154 -> 103).
 template <int METHOD, int NT, int NMAX>
 __device__ __forceinline__ void ring_dft(double2* buf, const RingLen& Ld) {
   if constexpr (METHOD == kAnyMethod) {
@@ -83,7 +97,7 @@ __device__ __forceinline__ void ring_dft(double2* buf, const RingLen& Ld) {
   }
 }
 
-template <int METHOD, bool UNIFORM, int NT, int NMAX>
+template <int METHOD, bool UNIFORM, RingPass PASS, int NT, int NMAX>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT < kDftNT ? 4 : 3))) void k_ring(RingArgs a) {
   constexpr int E = (NMAX + NT - 1) / NT;
   extern __shared__ unsigned char smem_raw[];
@@ -97,10 +111,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT < kDftNT 
   const double ph0 = a.phi0[ring];
   const long ofs = a.ofs[ring];
   const double2* g = a.G + ring;  // G[row][ring], row stride gstride
-  if (a.mode < 3) {
+  if constexpr (PASS != kToRows) {
     // conjugated spectrum for the inverse DFT: X[m mod n] = sum conj(G_m e^{i m phi0}) over the m that alias there
     const int mlo = a.spin ? -L : 0;
-    if (UNIFORM || n >= 2 * L + 1) {
+    if (PASS == kFullBand || n >= 2 * L + 1) {
       for (int k = threadIdx.x; k < n; k += NT) buf[k] = double2{0.0, 0.0};
       // The thread's rows (at most E: L - mlo < n <= NMAX) are loaded unconditionally, from rows
       // clamped to L, so that every load is in flight before the first LDS write.
@@ -131,7 +145,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT < kDftNT 
       // in LDS in order of m (the launch has room for max(L - mlo + 1, DFT values)); then every k adds its terms up, for
       // short rings split over P threads (a ring of four pixels has 2 lmax / 4 terms per k).  One loop over k and its
       // terms, each loaded when its turn came, made the polar rings the launch's whole time: 2047 HEALPix rings at
-      // nside 512, lmax 1000, took 347 us in three launches (one per DFT method), now 218 us.
+      // nside 512, lmax 1000, spin 2, took 295 us, with staged rows 166 and inlined transforms 117.
       const int nrow = L - mlo + 1;
       double2 gv[E];
 #pragma unroll
@@ -237,20 +251,35 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT < kDftNT 
 
 using RingKernel = void (*)(RingArgs);
 
-template <int CLASS>
+template <int CLASS, RingPass PASS>
 RingKernel ring_kernel(int method, bool uniform) {
   constexpr int NT = kRingNT[CLASS], NMAX = kRingNMax[CLASS];
-  if constexpr (CLASS == kRingClasses - 1) {
-    if (method == (int)DftMethod::Split) return uniform ? k_ring<3, true, NT, NMAX> : k_ring<3, false, NT, NMAX>;
+  constexpr int kDirect = (int)DftMethod::Direct, kRader = (int)DftMethod::Rader, kBlue = (int)DftMethod::Bluestein,
+                kSplit = (int)DftMethod::Split;
+  if constexpr (PASS != kFullBand) {  // (rings of several lengths take the kernel of any length)
+    if (!uniform) {
+      if constexpr (CLASS == kRingClasses - 1)
+        if (method == kSplit) return k_ring<kSplit, false, PASS, NT, NMAX>;
+      return method == kDirect ? k_ring<kDirect, false, PASS, NT, NMAX>
+             : method == kRader ? k_ring<kRader, false, PASS, NT, NMAX>
+             : method == kBlue ? k_ring<kBlue, false, PASS, NT, NMAX> : k_ring<kAnyMethod, false, PASS, NT, NMAX>;
+    }
   }
-  if (!uniform) return k_ring<kAnyMethod, false, NT, NMAX>;
-  if (method == (int)DftMethod::Direct) return k_ring<0, true, NT, NMAX>;
-  return method == (int)DftMethod::Rader ? k_ring<1, true, NT, NMAX> : k_ring<2, true, NT, NMAX>;
+  if constexpr (CLASS == kRingClasses - 1)
+    if (method == kSplit) return k_ring<kSplit, true, PASS, NT, NMAX>;
+  return method == kDirect ? k_ring<kDirect, true, PASS, NT, NMAX>
+         : method == kRader ? k_ring<kRader, true, PASS, NT, NMAX> : k_ring<kBlue, true, PASS, NT, NMAX>;
 }
 
+template <RingPass PASS>
 RingKernel ring_kernel(int cls, int method, bool uniform) {
-  return cls == 0 ? ring_kernel<0>(method, uniform)
-         : cls == 1 ? ring_kernel<1>(method, uniform) : ring_kernel<2>(method, uniform);
+  return cls == 0 ? ring_kernel<0, PASS>(method, uniform)
+         : cls == 1 ? ring_kernel<1, PASS>(method, uniform) : ring_kernel<2, PASS>(method, uniform);
+}
+
+RingKernel ring_kernel(RingPass pass, int cls, int method, bool uniform) {
+  return pass == kFullBand ? ring_kernel<kFullBand>(cls, method, uniform)
+         : pass == kAliased ? ring_kernel<kAliased>(cls, method, uniform) : ring_kernel<kToRows>(cls, method, uniform);
 }
 
 __global__ void k_sqrt_ll(int lmax, double* out) {
@@ -274,20 +303,11 @@ RingPlan::RingPlan(int lmax, int spin, const std::vector<double>& theta, const s
   }
   npix_ = 0;
   for (int i = 0; i < nring_; ++i) npix_ = std::max(npix_, ofs[i] + nph[i]);
-  // one DFT description per distinct ring length; rings grouped by workgroup size, the split DFTs apart
-  static_assert(kRingGroups == kRingClasses + 1, "one launch per workgroup size and one for the split DFTs");
+  // one DFT description per distinct ring length
   std::vector<int> lidx(nring_);
-  std::vector<std::vector<int>> by_group(kRingGroups);
   int longest = 0;
   for (int i = 0; i < nring_; ++i) {
     lidx[i] = dft_.add((int)nph[i], st);
-    const RingLen& d = dft_.at(lidx[i]);
-    const int values = ring_values(d, spin ? 2 * lmax + 1 : lmax + 1, 2 * lmax + 1);
-    const int cls = ring_class(d, values);
-    const int grp = d.method == (int)DftMethod::Split ? kRingClasses : cls;
-    by_group[grp].push_back(i);
-    // (the sums over aliased rows hold one value per thread)
-    lds_[grp] = std::max(lds_[grp], sizeof(double2) * (size_t)std::max(values, kRingNT[cls]));
     if (nph[i] > nph[longest]) longest = i;
   }
   method_ = (RingMethod)dft_.at(lidx[longest]).method;
@@ -295,29 +315,16 @@ RingPlan::RingPlan(int lmax, int spin, const std::vector<double>& theta, const s
   for (int i = 0; i < dft_.size(); ++i) lv.push_back(dft_.at(i));
   upload(lens_, lv);
   upload(lenidx_, lidx);
-  for (int m = 0; m < kRingGroups; ++m) {
-    nrings_m_[m] = (int)by_group[m].size();
-    if (nrings_m_[m]) upload(rings_[m], by_group[m]);
-    uniform_[m] = -1;
-    for (int i : by_group[m]) {
-      if (uniform_[m] == -1) uniform_[m] = lidx[i];
-      else if (uniform_[m] != lidx[i]) { uniform_[m] = -2; break; }
-    }
-  }
-  for (int cls = 0; cls < kRingClasses; ++cls)
-    for (int method = 0; method < (cls == kRingClasses - 1 ? kDftMethods : (int)DftMethod::Split); ++method)
-      for (bool uni : {false, true})
-        NUSHT_HIP(hipFuncSetAttribute((const void*)ring_kernel(cls, method, uni),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)(sizeof(double2) * kRingNMax[cls])));
+  nrows_ = spin ? 2 * lmax + 1 : lmax + 1;
+  gstride_ = nring_;
+  group_rings(lidx, true);
+  group_rings(lidx, false);
   upload(theta_, theta);
   upload(phi0_, phi0);
   upload(ofs_, ofs);
   if (!weight.empty()) upload(weight_, weight);
   tab_.tag = "ring";
   tab_.build(lmax, spin, theta, st);
-  nrows_ = spin ? 2 * lmax + 1 : lmax + 1;
-  gstride_ = nring_;
   G_.alloc(sizeof(double2) * (size_t)gstride_ * nrows_);
   coef_.alloc(legendre_coef_bytes(tab_, 1));
   sqll_.alloc(sizeof(double) * (lmax + 1));
@@ -327,18 +334,69 @@ RingPlan::RingPlan(int lmax, int spin, const std::vector<double>& theta, const s
   if (spin) legendre_autotune(tab_, 1, coef_.as<double2>(), G_.as<double2>(), gstride_, 1, st);  // E only
 }
 
+// Launches of one direction (to_rings: rows -> rings).  Rings are grouped by workgroup size and, above the smallest, by DFT
+// method: of the short rings of a ragged grid one launch takes all methods, since every launch lasts as long as its
+// slowest ring (HEALPix nside 32, lmax 64: 16 us, 26 with one launch per method), while long ones gain more from a
+// kernel of their own (nside 2048, lmax 2500, synthesis: 2.00 ms, 2.19 in one launch).
+void RingPlan::group_rings(const std::vector<int>& lidx, bool to_rings) {
+  const int band = 2 * lmax_ + 1;
+  std::vector<int> values(nring_);
+  int most = 0;
+  for (int i = 0; i < nring_; ++i) {
+    const RingLen& d = dft_.at(lidx[i]);
+    values[i] = to_rings ? ring_values(d, nrows_, band) : d.lds_values();
+    most = std::max(most, values[i]);
+  }
+  const bool few = nring_ <= kFewRings && most > kFewRingsValues;
+  std::map<int, std::set<int>> methods;  // of each size
+  const auto size_of = [&](int i) { return few ? std::max(1, ring_class(most)) : ring_class(values[i]); };
+  for (int i = 0; i < nring_; ++i)
+    if (dft_.at(lidx[i]).method != (int)DftMethod::Split) methods[size_of(i)].insert(dft_.at(lidx[i]).method);
+  std::map<std::pair<int, int>, std::vector<int>> launches;
+  for (int i = 0; i < nring_; ++i) {
+    int cls = size_of(i), method = dft_.at(lidx[i]).method;
+    if (method == (int)DftMethod::Split) cls = kRingClasses - 1;  // long rings only
+    else if (methods[cls].size() > 1 && (few || cls == 0)) method = kAnyMethod;
+    launches[{cls, method}].push_back(i);
+  }
+  for (const auto& [key, ids] : launches) {
+    RingGroup g;
+    g.cls = key.first;
+    g.method = key.second;
+    g.n = (int)ids.size();
+    bool one = true, full = true;
+    int v = kRingNT[g.cls];  // (the sums over aliased rows hold one value per thread)
+    for (int i : ids) {
+      one &= lidx[i] == lidx[ids[0]];
+      full &= dft_.at(lidx[i]).n >= band;
+      v = std::max(v, values[i]);
+    }
+    g.one = one ? lidx[ids[0]] : -1;
+    if (one) g.method = dft_.at(g.one).method;
+    g.pass = !to_rings ? kToRows : one && full ? kFullBand : kAliased;
+    g.lds = sizeof(double2) * (size_t)v;
+    // Rows that alias are staged in LDS if they fit.  One or two terms per value are as well read in turn where a ring
+    // fills a CU (3001 rings of 6000 pixels, lmax 3000, spin 2: 408 us, 442 staged).
+    g.stage = nrows_ <= kDftNMAX && !(one && g.cls == kRingClasses - 1 && dft_.at(g.one).n > lmax_);
+    upload(g.ids, ids);
+    NUSHT_HIP(hipFuncSetAttribute((const void*)ring_kernel((RingPass)g.pass, g.cls, g.method, one),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  (int)(sizeof(double2) * kRingNMax[g.cls])));
+    groups_.push_back(std::move(g));
+  }
+}
+
 size_t RingPlan::bytes() const {
   size_t b = tab_.bytes() + theta_.bytes() + phi0_.bytes() + ofs_.bytes() + weight_.bytes() + sqll_.bytes() +
              G_.bytes() + coef_.bytes() + lens_.bytes() + lenidx_.bytes();
   b += dft_.bytes();
-  for (int m = 0; m < kRingGroups; ++m) b += rings_[m].bytes();
+  for (const RingGroup& g : groups_) b += g.ids.bytes();
   return b;
 }
 
 void RingPlan::ring_pass(int mode, double* o0, double* o1, double* o2, hipStream_t st, const double* wt) {
   RingArgs a;
   a.lmax = lmax_; a.spin = spin_; a.gstride = gstride_; a.mode = mode;
-  a.stage = nrows_ <= kDftNMAX ? 1 : 0;
   a.lenidx = lenidx_.as<int>();
   a.lens = lens_.as<RingLen>();
   a.theta = theta_.as<double>(); a.phi0 = phi0_.as<double>(); a.ofs = ofs_.as<long>();
@@ -348,15 +406,13 @@ void RingPlan::ring_pass(int mode, double* o0, double* o1, double* o2, hipStream
   a.wt = wt;
   static const char* names[4] = {"ring_dft_synth_s0", "ring_dft_synth_spin", "ring_dft_pointing", "ring_dft_adjoint"};
   StageScope sc(names[mode], st);
-  for (int m = 0; m < kRingGroups; ++m) {
-    if (!nrings_m_[m]) continue;
-    a.rings = rings_[m].as<int>();
-    const bool uni = uniform_[m] >= 0 && dft_.at(uniform_[m]).n >= 2 * lmax_ + 1;
-    if (uni) a.one = dft_.at(uniform_[m]);
-    const int cls = std::min(m, kRingClasses - 1);
-    const int method = m == kRingClasses ? (int)DftMethod::Split : uni ? a.one.method : (int)DftMethod::Direct;
-    const RingKernel k = ring_kernel(cls, method, uni);
-    hipLaunchKernelGGL(k, dim3(nrings_m_[m]), dim3(kRingNT[cls]), lds_[m], st, a);
+  for (const RingGroup& g : groups_) {
+    if ((g.pass == kToRows) != (mode == 3)) continue;
+    a.rings = g.ids.as<int>();
+    a.stage = g.stage;
+    if (g.one >= 0) a.one = dft_.at(g.one);
+    hipLaunchKernelGGL(ring_kernel((RingPass)g.pass, g.cls, g.method, g.one >= 0), dim3(g.n), dim3(kRingNT[g.cls]),
+                       g.lds, st, a);
     NUSHT_LAUNCH_CHECK();
   }
 }
