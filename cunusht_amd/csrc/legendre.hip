@@ -6,8 +6,8 @@
 //               and arrive through the scalar cache (small transforms: as vector loads and DPP row
 //               broadcasts); the l-loop runs in two phases, first with underflow rescaling while any
 //               lane is still below 2^-300, then plain.
-//   adjoint   : the same waves; per-l sums over the lanes are formed in registers (halving steps over
-//               lane swaps) and added to the output with atomics, a last pass scales them.
+//   adjoint   : one wave per (m, one to four groups); per-l sums over the lanes are formed in registers (halving steps over
+//               lane swaps) and, unless one wave has them all, added to the output with atomics and scaled by a last pass.
 #include "legendre.h"
 
 #include "timing.h"
@@ -987,6 +987,7 @@ struct AdjArgs {
   const int* start;
   const double2* G;
   long sm, sr;
+  const double* cnorm;
   double2* alm;
 };
 
@@ -1003,8 +1004,11 @@ struct AdjArgs {
 // Times, ms, with the clearing and finishing passes (0.16 at lmax 4095): spin 2 lmax 4095 R = 1 / 2 / 3 / 4:
 // 13.4 / 10.2 / 9.3 / 9.6 (13.9 before), spin 0 6.1 / 4.2 / 3.65 / 3.7 (10.1 before); lmax 300 spin 2 0.040 / 0.047 /
 // 0.053 (0.131 before): few waves want the shorter l-step.
-template <int MODE, int R>
+// ALL: at most 64 ring pairs, so the wave has an m's whole sums and writes alm itself, without the passes before and
+// after (lmax 64, us: spin 0 16.8 -> 9.0, spin 2 19.5 -> 11.6; 10.7 and 16.2 in one workgroup per m with LDS sums).
+template <int MODE, int R, bool ALL = false>
 __global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
+  static_assert(!ALL || R == 1, "one group of ring pairs");
   constexpr bool SP = MODE != kScalar;
   constexpr int NA = MODE == kFull ? 4 : 2;  // doubles per (l, m)
   constexpr int K = 16 / NA;                 // l per lane sum
@@ -1016,8 +1020,19 @@ __global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
   const int L = a.lmax;
   if (m > L) return;
   const int l0 = l0_of(m, a.s);
-  if (l0 > L || sb * 64 * R >= a.nslot) return;
   const int lane = threadIdx.x;
+  const long nalm = (long)(L + 1) * (L + 2) / 2;
+  const long row = (long)m * (2 * L + 1 - m) / 2;  // of (l, m) = (0, m) in alm
+  const auto zero_below = [&](int l1) {  // the coefficients with l < l1
+    for (int l = m + lane; l < l1; l += 64) {
+      a.alm[row + l] = double2{0.0, 0.0};
+      if constexpr (MODE == kFull) a.alm[nalm + row + l] = double2{0.0, 0.0};
+    }
+  };
+  if constexpr (ALL) {
+    if (l0 > L) zero_below(L + 1);
+  }
+  if (l0 > L || sb * 64 * R >= a.nslot) return;
   const long base = a.mofs[m];
   const double* __restrict__ rec = reinterpret_cast<const double*>(a.rec + base) + (lane & 15);
 
@@ -1072,14 +1087,28 @@ __global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
   }
   lc = __builtin_amdgcn_readfirstlane(lc);
   lall = __builtin_amdgcn_readfirstlane(lall);
+  if constexpr (ALL) zero_below(lc);
   if (lc > L) return;
 
-  // where this lane's total goes (one lane of each quad writes)
+  // where this lane's total goes (one lane of each quad writes; ALL: the lane with Y.x has B's imaginary part, see below)
   const int wl = (lane >> 2) / NA, wc = (lane >> 2) % NA;
   const bool writer = (lane & 3) == 0;
-  const long nalm = (long)(L + 1) * (L + 2) / 2;
-  double* __restrict__ out = reinterpret_cast<double*>(
-      a.alm + (long)m * (2 * L + 1 - m) / 2 + l0 + wl + (wc >> 1) * nalm) + (wc & 1);
+  double* __restrict__ out = reinterpret_cast<double*>(a.alm + row + l0 + wl + (wc >> 1) * nalm) +
+                             ((wc & 1) ^ (ALL ? wc >> 1 : 0));
+  const double* __restrict__ cn = a.cnorm + base + wl;
+  // The sums of one coefficient -> alm, as in k_adjoint_finish (padded table: l may be past lmax).
+  const auto finished = [&](double t, int l) {
+    const double c = cn[l - l0];
+    if constexpr (MODE == kScalar) {
+      return m == 0 && wc == 1 ? 0.0 : c * t;
+    } else if constexpr (MODE == kGrad) {
+      return -0.5 * c * t;
+    } else {
+      const double u = dpp_mov<kDppRowRor8>(t);  // X and Y of a part are 8 lanes apart
+      const double X = ((a.s & 1) ? -c : c) * (wc < 2 ? t : u), Y = c * (wc < 2 ? u : t);
+      return wc < 2 ? -0.5 * (X + Y) : wc == 2 ? 0.5 * (X - Y) : -0.5 * (X - Y);
+    }
+  };
 
   // One chunk of 8 l.  SLOW: a group may join, some lane may be below range; FULL: all 8 l <= L.
   auto chunk = [&](int l, double rc, auto slow_tag, auto full_tag) {
@@ -1136,9 +1165,13 @@ __global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
         v[i * NA + 1] = X.y;
         if constexpr (MODE == kFull) { v[i * NA + 2] = Y.x; v[i * NA + 3] = Y.y; }
       });
-      const double total = wave_sums(v);
       const int lh = l + h * K;
-      if (writer && (FULL || lh + wl <= L)) atomicAdd(out + 2 * (lh - l0), total);
+      double total = wave_sums(v);
+      if constexpr (ALL) total = finished(total, lh);
+      if (writer && (FULL || lh + wl <= L)) {
+        if constexpr (ALL) out[2 * (lh - l0)] = total;
+        else atomicAdd(out + 2 * (lh - l0), total);
+      }
     });
   };
   auto any_under = [&]() {
@@ -1587,6 +1620,12 @@ static int adjoint_groups(int mode, int lmax, int ngroups) {
 template <int MODE>
 static void launch_adjoint(const LegendreTables& t, AdjArgs a, hipStream_t st) {
   const int L = t.lmax;
+  if (t.ngroups == 1) {
+    a.nsb = 1;
+    hipLaunchKernelGGL((k_adjoint<MODE, 1, true>), dim3(ceil_div(L + 1, kNumXcd) * kNumXcd), dim3(64), 0, st, a);
+    NUSHT_LAUNCH_CHECK();
+    return;
+  }
   const long n = (long)(L + 1) * (L + 2) / 2 * (MODE == kFull ? 2 : 1);
   hipLaunchKernelGGL(k_adjoint_clear, dim3((unsigned)std::min<long>(4096, (n + 255) / 256)), dim3(256), 0, st, a.alm, n);
   NUSHT_LAUNCH_CHECK();
@@ -1616,7 +1655,7 @@ void legendre_adjoint(const LegendreTables& t, int ncomp, const double2* G, long
   a.st_p = t.st_p.as<double2>();
   a.st_k = t.st_k.as<double2>();
   a.start = t.start.as<int>();
-  a.G = G; a.sm = sm; a.sr = sr; a.alm = alm;
+  a.G = G; a.sm = sm; a.sr = sr; a.alm = alm; a.cnorm = t.cnorm.as<double>();
   // the lmax that the adjoint is built and checked for
   NUSHT_REQUIRE(t.lmax <= (t.spin ? 5119 : 10239), kErrUnsupported, "legendre_adjoint: lmax too large");
   StageScope sc(t.n_adj.c_str(), st);
