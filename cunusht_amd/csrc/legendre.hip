@@ -1537,9 +1537,11 @@ static void legendre_synth_chunk(const LegendreTables& t, int nmaps, int ncomp, 
 
 int legendre_variant_count() { return kNumSynVariants; }
 
-// Waves of a one-group launch (m times ring groups) below which a table takes the row-broadcast synthesis unmeasured.
-// At lmax 255 (768 waves, spin 0) it takes 10 us against 22, at lmax 1000 (8008) 0.070 to 0.160 ms against 0.118 to
-// 0.218; between 20 us launches the measurement took the slower one in one process of four.
+// Waves of a one-group launch (m times ring groups) below which a table takes the row-broadcast synthesis without
+// measuring the others.  At lmax 255 (768 waves, spin 0) it takes 10 us against 22, at lmax 1000 (8008) 0.070 to
+// 0.160 ms against 0.118 to 0.218; between 20 us launches the measurement took the slower one in one process of four.
+// Few rings at a high lmax are the same case: 24 rings at lmax 4000 (4001 waves) 0.39 ms against 1.04 (spin 2), 0.22
+// against 0.66 (spin 0).
 constexpr long kRowWaves = 4096;
 
 void legendre_autotune(LegendreTables& t, int ncomp, double2* coef_ws, double2* G, long sm, long sr, hipStream_t st) {
@@ -1553,11 +1555,7 @@ void legendre_autotune(LegendreTables& t, int ncomp, double2* coef_ws, double2* 
   }
   const bool gr = t.spin > 0 && ncomp == 1;
   int& slot = gr ? t.variant_grad : t.variant;
-  // Few waves: the row broadcasts are up to twice as fast, while launches this short are not told apart by their times
-  if ((long)(t.lmax + 1) * t.ngroups < kRowWaves) {
-    slot = 0;
-    return;
-  }
+  const int nvar = (long)(t.lmax + 1) * t.ngroups < kRowWaves ? 1 : kNumSynVariants;
   // one measurement per (lmax, spin, ring pairs) and process
   static std::mutex mu;
   static std::map<std::tuple<int, int, int, int>, std::pair<int, float>> cache;
@@ -1581,7 +1579,7 @@ void legendre_autotune(LegendreTables& t, int ncomp, double2* coef_ws, double2* 
   int bestv = 0;
   const char* env = getenv("NUSHT_VERBOSE");
   const bool verbose = env && env[0] && env[0] != '0';
-  for (int v = 0; v < kNumSynVariants; ++v) {
+  for (int v = 0; v < nvar; ++v) {
     slot = v;
     legendre_synth(t, 1, ncomp, alm, 0, nullptr, coef_ws, G, sm, sr, 0, st);  // warm-up
     NUSHT_HIP(hipEventRecord(e0, st));
