@@ -259,8 +259,14 @@ __device__ __forceinline__ double rescaled_weight(double& mu, double& p, float& 
 // recursion values are real, the -m sums are conjugates of the +m ones: the kernel accumulates
 // sum W' mu_u and sum W' mu_v split by the parity of l - l0 (half the contraction of the E + B case) and
 // forms the four ring coefficients at the end.
-template <bool SP, int NB, int R, int CH, bool GR, int MINW>
-__global__ __launch_bounds__(64, MINW) void k_synth(SynthArgs a) {
+// Two maps (NB = 2) leave registers for one group per wave, and its waves wait for the coefficient stream again.  While
+// all of a launch's waves fit the GPU at once, blocks of WPB = 8 waves take neighbouring groups of one m, and seven of
+// them find its coefficients in the CU's scalar cache; a longer launch is better off with free blocks, for spin 0 of two
+// groups.  Two maps, ms, measured variant of the kernels before (2 or 4 l per chunk, blocks of 1, 4 or 8) / one wave per
+// block, 2 l per chunk / now: spin 0 lmax 511 0.061 / 0.078 / 0.054, 900 0.115 / 0.153 / 0.116, 2047 0.88 / 0.98 / 0.68,
+// 4095 5.69 / 7.00 / 4.14; spin 2 lmax 511 0.100 / 0.094 / 0.091, 900 0.214 / 0.233 / 0.211, 2047 1.66 / 1.44 / 1.44.
+template <bool SP, int NB, int R, int CH, bool GR, int MINW, int WPB = 1>
+__global__ __launch_bounds__(64 * WPB, MINW) void k_synth(SynthArgs a) {
   static_assert(SP || !GR, "the gradient-only contraction is a spin-s case");
   static_assert(kRescaleL % CH == 0, "rescale checks fall on chunk starts");
   constexpr int K = (SP && !GR) ? 2 * NB : NB;
@@ -270,13 +276,13 @@ __global__ __launch_bounds__(64, MINW) void k_synth(SynthArgs a) {
   const int blk = blockIdx.x;
   const int j = blk / kNumXcd;
   const int m = (blk - j * kNumXcd) + kNumXcd * (j / a.nsb);
-  const int sb = j % a.nsb;
+  const int sb = (j % a.nsb) * WPB + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int L = a.lmax;
   if (m > L) return;
   const int l0 = l0_of(m, a.s);
   // the launch may carry empty slot groups (odd block count per m, see launch_synth)
   if (l0 > L || sb * 64 * R >= a.nslot) return;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
   const int ng = (a.nslot + 63) >> 6;
 
   double x[R], mu_u[R], mu_v[R], pu[R], pv[R];
@@ -1350,10 +1356,15 @@ size_t legendre_coef_bytes(const LegendreTables& t, int nmaps) {
 }
 
 // Synthesis variants of one map, in order of the launch size they suit: k_synth_row, k_synth with few and with more
-// ring groups per wave; the autotuner picks one per table.  Launches of two maps take one group per wave
-// (k_synth<.., 2, 1, 2, ..>: the second map's accumulators take the registers of a second group).
+// ring groups per wave; the autotuner picks one per table.  Launches of two maps go by their waves (kTwoMapWaves).
 static const char* const kSynVariants[] = {"row broadcasts", "few groups per wave", "more groups per wave"};
 constexpr int kNumSynVariants = 3;
+
+// Waves of 64 ring pairs (m times ring groups) from which launches of two maps take free blocks, spin 0 two groups per
+// wave: about those the GPU holds (256 CUs, 4 SIMDs, 8 waves).  Blocks of 8 waves / free blocks, ms: lmax 900 (7208 waves)
+// spin 0 0.115 / 0.129, spin 2 0.210 / 0.231; lmax 1000 (9009) 0.148 / 0.163, 0.27 / 0.27; lmax 1200 (12010) 0.237 / 0.209,
+// 0.42 / 0.39.
+constexpr long kTwoMapWaves = 10000;
 
 template <bool SP, int NB, bool GR = false>
 static void launch_synth(const SynthArgs& a, int variant, hipStream_t st) {
@@ -1366,7 +1377,15 @@ static void launch_synth(const SynthArgs& a, int variant, hipStream_t st) {
     return dim3((unsigned)(b.nsb * chains * ceil_div(a.lmax + 1, kNumXcd) * kNumXcd));
   };
   if constexpr (NB > 1) {
-    hipLaunchKernelGGL((k_synth<SP, NB, 1, 2, GR, 1>), blocks(1, 1), dim3(64), 0, st, b);
+    constexpr int CH = SP ? 2 : 4;
+    if ((long)(a.lmax + 1) * ceil_div(a.nslot, 64) < kTwoMapWaves) {
+      const dim3 grid = blocks(8, 1);
+      hipLaunchKernelGGL((k_synth<SP, NB, 1, CH, GR, 1, 8>), grid, dim3(64 * 8), 0, st, b);
+    } else {
+      constexpr int R = SP ? 1 : 2;
+      const dim3 grid = blocks(R, 1);
+      hipLaunchKernelGGL((k_synth<SP, NB, R, CH, GR, 1>), grid, dim3(64), 0, st, b);
+    }
   } else if (variant == 0) {
     constexpr int MODE = !SP ? kScalar : GR ? kGrad : kFull;
     const dim3 grid = blocks(1, SP ? 2 : 1);
