@@ -46,7 +46,7 @@ struct LegendreTables {
   std::string n_prep, n_synth, n_adj;
   int chunk = 2;          // maps per synthesis launch (VALU kernels)
   bool mfma = true;       // batches of >= 3 maps on the matrix cores (NUSHT_LEGENDRE_MFMA=0 turns it off)
-  int variant = -1;       // synthesis kernel variant (-1: default); set by legendre_autotune
+  int variant = -1;       // synthesis kernel variant (-1: by size); set by legendre_autotune
   int variant_grad = -1;  // the same for the E-only (gradient) contraction of spin-s tables
   float tuned_ms = 0.f;
 

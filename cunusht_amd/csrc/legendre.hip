@@ -1509,6 +1509,16 @@ static void legendre_synth_mfma(const LegendreTables& t, int nmaps, int ncomp, c
   NUSHT_LAUNCH_CHECK();
 }
 
+// Variant of a table that was not measured (point sets: no mirrored rings, so up to 64 points per group).  Spin s,
+// points at lmax, us, row broadcasts / few / more groups: 300 at 2000 390 / 471 / 540, 1000 at 300 39 / 51 / 57, 1000 at
+// 1000 306 / 248 / 302, 700 at 2000 757 / 655 / 699, 3000 at 1000 806 / 647 / 629, 1000 at 4000 3967 / 3858 / 3033.  Spin 0
+// is within 15 % of its best with row broadcasts, 1.3 to 2 times ahead below 1000 points.
+static int untuned_variant(const LegendreTables& t) {
+  const long waves = (long)(t.lmax + 1) * t.ngroups;
+  if (t.spin == 0 || t.ngroups < 8 || waves < 12000) return 0;
+  return waves < 40000 ? 1 : 2;
+}
+
 static void legendre_synth_chunk(const LegendreTables& t, int nmaps, int ncomp, const double2* alm,
                                  long alm_stride_map, const double* fl, double2* coef_ws, double2* G, long sm, long sr,
                                  long smap, hipStream_t st) {
@@ -1537,7 +1547,7 @@ static void legendre_synth_chunk(const LegendreTables& t, int nmaps, int ncomp, 
   const bool sp = t.spin > 0;
   const bool gr = sp && ncomp == 1;  // E only: the gradient-only contraction
   const int tv = gr ? t.variant_grad : t.variant;
-  const int var = (tv >= 0 && tv < kNumSynVariants) ? tv : 0;
+  const int var = (tv >= 0 && tv < kNumSynVariants) ? tv : untuned_variant(t);
   StageScope sc(t.n_synth.c_str(), st);
   switch (nbpad) {  // the kernel's NB must equal the coefficient stride written by k_prep
     case 1:

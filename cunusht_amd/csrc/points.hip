@@ -70,7 +70,6 @@ PointPlan::PointPlan(int lmax, int spin, const std::vector<double>& theta, hipSt
   nrows_ = spin ? 2 * lmax + 1 : lmax + 1;
   G_.alloc(sizeof(double2) * (size_t)nrows_ * npts_);
   coef_.alloc(legendre_coef_bytes(tab_, 1));
-  tab_.variant = 0;
 }
 
 void PointPlan::synthesis(const double2* alm, int ncomp, const double* phi, const double* gamma, double* out0,
