@@ -502,8 +502,9 @@ __device__ __forceinline__ void row_fma2(double2& acc, double c, double w) {
 // table, 4 or 8 of the map's), three chunks of 8 l deep, and reach the arithmetic as DPP row broadcasts; the two
 // chains run side by side in two waves.  With the coefficient preparation, ms, against the faster of k_synth with few
 // and with more groups: lmax 255 spin 2 0.033 -> 0.015, spin-1 gradient 0.027 -> 0.017, spin 0 0.022 -> 0.013;
-// lmax 1000 0.218 -> 0.160, 0.182 -> 0.125, 0.118 -> 0.070.  From lmax 1500 on (spin s) k_synth is the faster one
-// (two broadcasts per l and chain less): lmax 4095 spin 2 6.9 here, 4.8 there.
+// lmax 1000 0.218 -> 0.160, 0.182 -> 0.125, 0.118 -> 0.070.  For spin s k_synth is the faster one from lmax 1200 on
+// (two broadcasts per l and chain less): kernel alone, spin 2, here / few / more groups, lmax 1200 0.291 / 0.292 / 0.346,
+// 1500 0.53 / 0.49 / 0.52, 2047 1.16 / 1.04 / 1.07, 4095 7.5 / 7.1 / 6.1; spin 0 4095 2.49 / 3.23 / 2.74.
 template <int MODE>
 __global__ __launch_bounds__(64) void k_synth_row(SynthArgs a) {
   constexpr bool SP = MODE != kScalar;
@@ -1573,6 +1574,17 @@ int legendre_variant_count() { return kNumSynVariants; }
 // against 0.66 (spin 0).
 constexpr long kRowWaves = 4096;
 
+// Coefficients to measure on, of order one: on zeros the clock runs higher (2.33 GHz at lmax 4095, 2.05 on data), by
+// more for the denser kernels.  In three processes each over lmax 64 to 4095, measured on zeros and one kernel after the
+// other the tuner took row broadcasts at lmax 1500 spin 2 (0.51 ms, few groups 0.47) in two and more groups at lmax 4095
+// spin 0 (2.73 ms, row broadcasts 2.45) in one; on data, with every kernel run before the first is timed, in none.
+__global__ void k_tuning_alm(double2* __restrict__ alm, long n) {
+  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+    const unsigned h = (unsigned)i * 2654435761u;
+    alm[i] = double2{(h >> 16) * 0x1p-15 - 1.0, (h & 0xffffu) * 0x1p-15 - 1.0};
+  }
+}
+
 void legendre_autotune(LegendreTables& t, int ncomp, double2* coef_ws, double2* G, long sm, long sr, hipStream_t st) {
   // NUSHT_LEGENDRE_VARIANT=k fixes the variant (tests run every variant this way)
   if (const char* fv = getenv("NUSHT_LEGENDRE_VARIANT"); fv && fv[0]) {
@@ -1598,8 +1610,11 @@ void legendre_autotune(LegendreTables& t, int ncomp, double2* coef_ws, double2* 
       return;
     }
   }
-  DevBuf dummy(sizeof(double2) * (size_t)(t.lmax + 1) * (t.lmax + 2) / 2 * ncomp);
-  NUSHT_HIP(hipMemsetAsync(dummy.get(), 0, dummy.bytes(), st));
+  const long nalm = (long)(t.lmax + 1) * (t.lmax + 2) / 2 * ncomp;
+  DevBuf dummy(sizeof(double2) * (size_t)nalm);
+  hipLaunchKernelGGL(k_tuning_alm, dim3((unsigned)std::min<long>(4096, ceil_div(nalm, 256L))), dim3(256), 0, st,
+                     dummy.as<double2>(), nalm);
+  NUSHT_LAUNCH_CHECK();
   const double2* alm = dummy.as<double2>();
   hipEvent_t e0, e1;
   NUSHT_HIP(hipEventCreate(&e0));
@@ -1608,9 +1623,12 @@ void legendre_autotune(LegendreTables& t, int ncomp, double2* coef_ws, double2* 
   int bestv = 0;
   const char* env = getenv("NUSHT_VERBOSE");
   const bool verbose = env && env[0] && env[0] != '0';
+  for (int v = 0; v < nvar; ++v) {  // all of them first, or the one timed first is timed while the clock settles
+    slot = v;
+    legendre_synth(t, 1, ncomp, alm, 0, nullptr, coef_ws, G, sm, sr, 0, st);
+  }
   for (int v = 0; v < nvar; ++v) {
     slot = v;
-    legendre_synth(t, 1, ncomp, alm, 0, nullptr, coef_ws, G, sm, sr, 0, st);  // warm-up
     NUSHT_HIP(hipEventRecord(e0, st));
     for (int k = 0; k < 2; ++k) legendre_synth(t, 1, ncomp, alm, 0, nullptr, coef_ws, G, sm, sr, 0, st);
     NUSHT_HIP(hipEventRecord(e1, st));
