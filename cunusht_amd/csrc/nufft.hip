@@ -439,8 +439,12 @@ __device__ __forceinline__ void interp_mark_bad(const InterpArgs<T>& a) {
 }
 
 // Points per tile that the interpolation orders by bank class in LDS (tiles with more keep the binned order): 4 KiB of
-// 16-bit entries, and full maps on ragged grids reach 1200 points per tile near the equator.
+// 16-bit entries, and full maps on ragged grids reach 1200 points per tile near the equator.  Widths below
+// kInterpSortMinW keep the binned order too: ordering costs their few reads more than the conflicts (FP32, ordered / not,
+// us: w = 5, lmax 1024 4M points spin 0 96 / 70, lmax 700 100 000 points 15.0 / 12.4; FP64 w = 7, lmax 700 1M points
+// 50 / 44).
 constexpr int kInterpSortCap = 2048;
+constexpr int kInterpSortMinW = 8;
 
 // One workgroup per fine-grid tile: the tile plus its (W-1)-cell halo is staged in LDS once and
 // every point binned to the tile is interpolated from it (fully unrolled W x W footprint).
@@ -474,7 +478,7 @@ __global__ __launch_bounds__(256) void k_interp_w(InterpArgs<T> a) {
   int* ccnt = reinterpret_cast<int*>(smem_raw + sizeof(T2) * (size_t)tw * th);  // [16] class counts, then starts
   unsigned short* order = reinterpret_cast<unsigned short*>(ccnt + 16);            // [kInterpSortCap]
   const int n = s1 - s0;
-  const bool sorted = n <= kInterpSortCap;
+  const bool sorted = W >= kInterpSortMinW && n <= kInterpSortCap;
   if (sorted && threadIdx.x < 16) ccnt[threadIdx.x] = 0;
   const int tile_r = tb / a.ntc, tile_c = tb - (tb / a.ntc) * a.ntc;
   const int r0 = tile_r * a.tr, c0 = tile_c * a.tc;
@@ -518,7 +522,7 @@ __global__ __launch_bounds__(256) void k_interp_w(InterpArgs<T> a) {
     lr = i0 - a.row_lo - r0;
     lc = j0 - c0;
   };
-  if (sorted) {
+  if (sorted) {  // (never for the narrow widths, at compile time)
     constexpr int EI = kInterpSortCap / 256, EB = 4;
     int cls[EI], rank[EI];
 #pragma unroll
@@ -2005,8 +2009,8 @@ void NufftPlan::type2_impl(const double2* G, long sm, const double* gamma, doubl
                    grid_.as<T2>(), gamma, ore, oim};
   StageScope sc("nufft_interp", st);
   // tile, then (templated widths) the class counts and the point order
-  const size_t tlds = sizeof(T2) * (size_t)(tile_r_ + p.w) * (tile_c_ + p.w) + sizeof(int) * 16 +
-                      sizeof(unsigned short) * kInterpSortCap;
+  const size_t tlds = sizeof(T2) * (size_t)(tile_r_ + p.w) * (tile_c_ + p.w) +
+                      (p.w >= kInterpSortMinW ? sizeof(int) * 16 + sizeof(unsigned short) * kInterpSortCap : 0);
   launch_interp<T, 2>(p.w, dim3(ntiles + 1), tlds, st, ia);  // + 1: the workgroup for out-of-range points
   NUSHT_LAUNCH_CHECK();
 }
