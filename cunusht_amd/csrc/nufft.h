@@ -87,6 +87,7 @@ class NufftPlan {
   int rows_cap_ = 0;               // its LDS point records per pass
   int rows_seg_ = 1;               // tiles one workgroup walks down a column strip
   int ntile_r_ = 0, ntile_c_ = 0;
+  int cursor_ofs_ = 0;             // where the scatter's cursors start in tile_cnt_
   // tables
   DevBuf deconv_;                  // double[lmax+1] : 1 / psi_hat(k)
   DevBuf kpoly_;                   // T[(poly_deg+1) * w] kernel polynomials, degree-major
@@ -98,7 +99,7 @@ class NufftPlan {
   DevBuf pts_;                     // double2[npts_max] sorted points, positions in fine cells along theta and phi
   DevBuf idx_;                     // int[npts_max] original index of sorted point
   DevBuf tile_start_;              // int[ntiles + 1]
-  DevBuf tile_cnt_;                // int[ntiles + 1] counts, an error counter, int[ntiles + 1] scatter cursors
+  DevBuf tile_cnt_;                // int[ntiles + 1] counts, an error counter; scatter cursors int[ntiles + 1]
   DevBuf key_;                     // int[npts_max] tile of each point
   DevBuf scan_tmp_;                // hipcub scan temp storage
   size_t scan_tmp_bytes_ = 0;
