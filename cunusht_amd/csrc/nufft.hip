@@ -1388,7 +1388,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DM <= 12 ? 
         Rec r0 = record(g), r1 = record(g + 1);
         T kt, kp;
         horner2<DM, DM>(cf, r0.u.x, r0.u.y, kt, kp);
-#pragma unroll 2
         for (; g < gend; ++g) {
           const double wt = (double)lane_read(kt, 4 * ((lane & 48) + ((l16 - (r0.off >> 4)) & 15)));
           const double wp = (double)lane_read(kp, 4 * ((lane & 48) + ((l16 - r0.off) & 15)));
