@@ -998,6 +998,20 @@ struct AdjArgs {
   double2* alm;
 };
 
+// The sums over ring pairs -> alm, c the coefficient's norm (see k_adjoint).
+template <int MODE>
+__device__ __forceinline__ double2 adjoint_coef(int m, double c, double2 t) {
+  if constexpr (MODE == kScalar) return double2{c * t.x, m == 0 ? 0.0 : c * t.y};
+  else return cscale(t, -0.5 * c);
+}
+__device__ __forceinline__ void adjoint_coef(int s, double c, double2 x, double2 y, double2& e, double2& b) {
+  const double2 X = cscale(x, (s & 1) ? -c : c), Y = cscale(y, c);
+  e = double2{-0.5 * (X.x + Y.x), -0.5 * (X.y + Y.y)};
+  b = double2{-0.5 * (X.y - Y.y), 0.5 * (X.x - Y.x)};
+}
+
+constexpr int kAdjointAllWaves = 4;  // of a workgroup that holds all of an m's waves
+
 // One wave per (m, R groups of 64 ring pairs), as in the synthesis: every wave runs its own l-range, so polar groups,
 // which contribute late or never, hold nobody up.  (One workgroup per m with all its ring pairs and an LDS sum per l
 // filled a CU at lmax 4095 and waited for its equatorial waves.)  Per K l the wave adds up its ring pairs' products in
@@ -1011,11 +1025,12 @@ struct AdjArgs {
 // Times, ms, with the clearing and finishing passes (0.16 at lmax 4095): spin 2 lmax 4095 R = 1 / 2 / 3 / 4:
 // 13.4 / 10.2 / 9.3 / 9.6 (13.9 before), spin 0 6.1 / 4.2 / 3.65 / 3.7 (10.1 before); lmax 300 spin 2 0.040 / 0.047 /
 // 0.053 (0.131 before): few waves want the shorter l-step.
-// ALL: at most 64 ring pairs, so the wave has an m's whole sums and writes alm itself, without the passes before and
-// after (lmax 64, us: spin 0 16.8 -> 9.0, spin 2 19.5 -> 11.6; 10.7 and 16.2 in one workgroup per m with LDS sums).
+// ALL: the waves of one m form a workgroup and keep their totals in LDS; it adds them up in wave order and writes alm
+// itself, without the passes before and after, and repeats bit for bit.  Us, with atomics and three launches / now: spin 2
+// lmax 64 19.7 / 10.9, 300 47 / 31, 511 86 / 87, 700 173 / 137, 766 198 / 192; spin 0 35 / 19 at 300, 88 / 68 at 700.
 template <int MODE, int R, bool ALL = false>
-__global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
-  static_assert(!ALL || R == 1, "one group of ring pairs");
+__global__ __launch_bounds__(ALL ? 64 * kAdjointAllWaves : 64) void k_adjoint(AdjArgs a) {
+  extern __shared__ double adj_sums[];  // ALL: [wave][l - l0][NA]
   constexpr bool SP = MODE != kScalar;
   constexpr int NA = MODE == kFull ? 4 : 2;  // doubles per (l, m)
   constexpr int K = 16 / NA;                 // l per lane sum
@@ -1023,23 +1038,16 @@ __global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
   const int blk = blockIdx.x;
   const int j = blk / kNumXcd;
   const int m = (blk - j * kNumXcd) + kNumXcd * (j / a.nsb);
-  const int sb = j % a.nsb;
+  const int wave = ALL ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
+  const int sb = ALL ? wave : j % a.nsb;
   const int L = a.lmax;
   if (m > L) return;
   const int l0 = l0_of(m, a.s);
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
   const long nalm = (long)(L + 1) * (L + 2) / 2;
   const long row = (long)m * (2 * L + 1 - m) / 2;  // of (l, m) = (0, m) in alm
-  const auto zero_below = [&](int l1) {  // the coefficients with l < l1
-    for (int l = m + lane; l < l1; l += 64) {
-      a.alm[row + l] = double2{0.0, 0.0};
-      if constexpr (MODE == kFull) a.alm[nalm + row + l] = double2{0.0, 0.0};
-    }
-  };
-  if constexpr (ALL) {
-    if (l0 > L) zero_below(L + 1);
-  }
-  if (l0 > L || sb * 64 * R >= a.nslot) return;
+  const int nl = L + 1 - l0;
+  if (!ALL && (l0 > L || sb * 64 * R >= a.nslot)) return;
   const long base = a.mofs[m];
   const double* __restrict__ rec = reinterpret_cast<const double*>(a.rec + base) + (lane & 15);
 
@@ -1056,7 +1064,7 @@ __global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const int g = sb * R + r;
-    lst[r] = __builtin_amdgcn_readfirstlane(g < a.ngroups ? a.start[(long)m * a.ngroups + g] : L + 1);
+    lst[r] = __builtin_amdgcn_readfirstlane(g < a.ngroups && nl > 0 ? a.start[(long)m * a.ngroups + g] : L + 1);
     lc = min(lc, lst[r]);
     if (lst[r] <= L) lall = max(lall, lst[r]);
     const int slot = g * 64 + lane;
@@ -1094,28 +1102,15 @@ __global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
   }
   lc = __builtin_amdgcn_readfirstlane(lc);
   lall = __builtin_amdgcn_readfirstlane(lall);
-  if constexpr (ALL) zero_below(lc);
-  if (lc > L) return;
+  if (!ALL && lc > L) return;
 
-  // where this lane's total goes (one lane of each quad writes; ALL: the lane with Y.x has B's imaginary part, see below)
+  // where this lane's total goes (one lane of each quad writes)
   const int wl = (lane >> 2) / NA, wc = (lane >> 2) % NA;
   const bool writer = (lane & 3) == 0;
-  double* __restrict__ out = reinterpret_cast<double*>(a.alm + row + l0 + wl + (wc >> 1) * nalm) +
-                             ((wc & 1) ^ (ALL ? wc >> 1 : 0));
-  const double* __restrict__ cn = a.cnorm + base + wl;
-  // The sums of one coefficient -> alm, as in k_adjoint_finish (padded table: l may be past lmax).
-  const auto finished = [&](double t, int l) {
-    const double c = cn[l - l0];
-    if constexpr (MODE == kScalar) {
-      return m == 0 && wc == 1 ? 0.0 : c * t;
-    } else if constexpr (MODE == kGrad) {
-      return -0.5 * c * t;
-    } else {
-      const double u = dpp_mov<kDppRowRor8>(t);  // X and Y of a part are 8 lanes apart
-      const double X = ((a.s & 1) ? -c : c) * (wc < 2 ? t : u), Y = c * (wc < 2 ? u : t);
-      return wc < 2 ? -0.5 * (X + Y) : wc == 2 ? 0.5 * (X - Y) : -0.5 * (X - Y);
-    }
-  };
+  double* __restrict__ out = reinterpret_cast<double*>(a.alm + row + l0 + wl + (wc >> 1) * nalm) + (wc & 1);
+  double* sums = adj_sums + wave * nl * NA;
+  if constexpr (ALL)
+    for (int i = lane; i < min(lc - l0, nl) * NA; i += 64) sums[i] = 0.0;
 
   // One chunk of 8 l.  SLOW: a group may join, some lane may be below range; FULL: all 8 l <= L.
   auto chunk = [&](int l, double rc, auto slow_tag, auto full_tag) {
@@ -1172,11 +1167,10 @@ __global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
         v[i * NA + 1] = X.y;
         if constexpr (MODE == kFull) { v[i * NA + 2] = Y.x; v[i * NA + 3] = Y.y; }
       });
+      const double total = wave_sums(v);
       const int lh = l + h * K;
-      double total = wave_sums(v);
-      if constexpr (ALL) total = finished(total, lh);
       if (writer && (FULL || lh + wl <= L)) {
-        if constexpr (ALL) out[2 * (lh - l0)] = total;
+        if constexpr (ALL) sums[(lh - l0) * NA + (lane >> 2)] = total;
         else atomicAdd(out + 2 * (lh - l0), total);
       }
     });
@@ -1190,7 +1184,8 @@ __global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
   using T_ = std::true_type;
   using F_ = std::false_type;
   auto load = [&](int l) { return rec[2 * (long)(l - l0)]; };
-  double b0 = load(lc), b1 = load(lc + CH);
+  double b0 = 0.0, b1 = 0.0;
+  if (lc <= L) { b0 = load(lc); b1 = load(lc + CH); }
   while (lc <= L && (lc <= lall || any_under())) {
     const double b2 = load(lc + 2 * CH);
     if (lc + CH - 1 <= L) chunk(lc, b0, T_{}, T_{});
@@ -1212,6 +1207,27 @@ __global__ __launch_bounds__(64) void k_adjoint(AdjArgs a) {
     lc += CH;
   }
   if (lc <= L) chunk(lc, b0, F_{}, F_{});
+  if constexpr (ALL) {
+    __syncthreads();
+    const int nw = blockDim.x >> 6;
+    for (int l = m + (int)threadIdx.x; l <= L; l += blockDim.x) {
+      double2* e = a.alm + row + l;
+      if (l < l0) {
+        e[0] = double2{0.0, 0.0};
+        if constexpr (MODE == kFull) e[nalm] = double2{0.0, 0.0};
+        continue;
+      }
+      double t[NA];
+#pragma unroll
+      for (int k = 0; k < NA; ++k) t[k] = 0.0;
+      for (int w = 0; w < nw; ++w)
+#pragma unroll
+        for (int k = 0; k < NA; ++k) t[k] += adj_sums[(w * nl + l - l0) * NA + k];
+      const double c = a.cnorm[base + l - l0];
+      if constexpr (MODE == kFull) adjoint_coef(a.s, c, double2{t[0], t[1]}, double2{t[2], t[3]}, e[0], e[nalm]);
+      else e[0] = adjoint_coef<MODE>(m, c, double2{t[0], t[1]});
+    }
+  }
 }
 
 __global__ void k_adjoint_clear(double2* __restrict__ p, long n) {
@@ -1232,16 +1248,8 @@ __global__ __launch_bounds__(256) void k_adjoint_finish(int L, int s, const long
     for (int l = l0 + blockIdx.x * blockDim.x + threadIdx.x; l <= L; l += gridDim.x * blockDim.x) {
       const double c = cnorm[mofs[m] + (l - l0)];
       double2* e = alm + mbase + l;
-      if constexpr (MODE == kScalar) {
-        *e = double2{c * e->x, m == 0 ? 0.0 : c * e->y};
-      } else if constexpr (MODE == kGrad) {
-        *e = cscale(*e, -0.5 * c);
-      } else {
-        const double sc = (s & 1) ? -c : c;
-        const double2 X = cscale(*e, sc), Y = cscale(e[nalm], c);
-        *e = double2{-0.5 * (X.x + Y.x), -0.5 * (X.y + Y.y)};
-        e[nalm] = double2{-0.5 * (X.y - Y.y), 0.5 * (X.x - Y.x)};
-      }
+      if constexpr (MODE == kFull) adjoint_coef(s, c, *e, e[nalm], *e, e[nalm]);
+      else *e = adjoint_coef<MODE>(m, c, *e);
     }
   }
 }
@@ -1648,13 +1656,12 @@ void legendre_autotune(LegendreTables& t, int ncomp, double2* coef_ws, double2* 
   cache[key] = {bestv, best / 2};
 }
 
-// Ring groups per wave of the adjoint.  Up to 384 ring pairs (512 for spin 0) one or two waves hold an m: their sums on a
-// cleared output come out the same in either order, so the adjoint repeats bit for bit (with one group per wave, three or
-// more waves at lmax 300 / 511 / 766: spin 2 0.048 / 0.086 / 0.198 ms, now 0.054 / 0.108 / 0.198).  Above, three or more
-// waves add in any order, and the choice is by time: three groups once a launch with three has kAdjointMinWaves waves; below it a
-// SIMD has one or two waves, and the shorter l-step of one group is worth more than the shared lane sums.  Measured, ms,
-// one / three groups: lmax 700 spin 0 0.090 / 0.096, spin 2 0.167 / 0.174 (1402 waves); lmax 850 0.120 / 0.122,
-// 0.224 / 0.231 (2553); lmax 1000 0.170 / 0.148, 0.296 / 0.276 (3003).
+// Ring groups per wave of the adjoint where its waves add to the output.  Up to 384 ring pairs (512 for spin 0) one or two
+// waves hold an m: their sums on a cleared output come out the same in either order, so the adjoint repeats bit for bit.
+// Above, three or more waves add in any order, and the choice is by time: three groups once a launch with three has
+// kAdjointMinWaves waves; below it a SIMD has one or two waves, and the shorter l-step of one group is worth more than the
+// shared lane sums.  Measured, ms, one / three groups: lmax 700 spin 0 0.090 / 0.096, spin 2 0.167 / 0.174 (1402 waves);
+// lmax 850 0.120 / 0.122, 0.224 / 0.231 (2553); lmax 1000 0.170 / 0.148, 0.296 / 0.276 (3003).
 constexpr long kAdjointMinWaves = 2600;
 
 static int adjoint_groups(int mode, int lmax, int ngroups) {
@@ -1665,9 +1672,17 @@ static int adjoint_groups(int mode, int lmax, int ngroups) {
 template <int MODE>
 static void launch_adjoint(const LegendreTables& t, AdjArgs a, hipStream_t st) {
   const int L = t.lmax;
-  if (t.ngroups == 1) {
+  // All of an m's waves in one workgroup, up to 512 ring pairs and as long as their totals in LDS leave a CU five waves (us,
+  // in LDS / added to the output: 24 rings at lmax 1000 spin 2, five waves, 98 / 131; 256 rings at lmax 2000 spin 0, four,
+  // 307 / 247); one group per wave up to four, two above (one / two: spin 2 lmax 300 31 / 38, 511 97 / 87, 700 182 / 137).
+  const int RA = t.ngroups <= kAdjointAllWaves ? 1 : 2, nw = ceil_div(t.ngroups, RA);
+  const size_t lds = sizeof(double) * (MODE == kFull ? 4 : 2) * (size_t)nw * (L + 1);
+  if (nw <= kAdjointAllWaves && nw * (160 * 1024 / lds) >= 5) {
     a.nsb = 1;
-    hipLaunchKernelGGL((k_adjoint<MODE, 1, true>), dim3(ceil_div(L + 1, kNumXcd) * kNumXcd), dim3(64), 0, st, a);
+    const auto kern = RA == 1 ? k_adjoint<MODE, 1, true> : k_adjoint<MODE, 2, true>;
+    if (lds > 64 * 1024)
+      NUSHT_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(kern, dim3((unsigned)(ceil_div(L + 1, kNumXcd) * kNumXcd)), dim3(64 * nw), lds, st, a);
     NUSHT_LAUNCH_CHECK();
     return;
   }
