@@ -91,7 +91,7 @@ void legendre_autotune(LegendreTables& t, int ncomp, double2* coef_ws, double2* 
 
 // Adjoint: G -> alm (exact transpose of legendre_synth under the real-field alm inner product).
 // For spin 0 only rows m = 0..lmax are read (the field is real); m = 0 imaginary parts are dropped.
-// alm (device memory) is the only storage: above 64 ring pairs it is cleared, summed into with FP64 atomics and scaled.
+// alm (device memory) is the only storage; with more than 512 ring pairs it is summed into with FP64 atomics.
 void legendre_adjoint(const LegendreTables& t, int ncomp, const double2* G, long g_stride_m, long g_stride_r,
                       double2* alm, hipStream_t st);
 

@@ -7,7 +7,8 @@
 //               broadcasts); the l-loop runs in two phases, first with underflow rescaling while any
 //               lane is still below 2^-300, then plain.
 //   adjoint   : one wave per (m, one to four groups); per-l sums over the lanes are formed in registers (halving steps over
-//               lane swaps) and, unless one wave has them all, added to the output with atomics and scaled by a last pass.
+//               lane swaps) and added up over an m's waves in LDS (up to 512 ring pairs) or, with atomics, in the output,
+//               which a last pass scales.
 #include "legendre.h"
 
 #include "timing.h"
