@@ -261,7 +261,7 @@ __device__ __forceinline__ void fft_stage(c2_t<T>* buf, int n, int ns, const c2_
 // GENERIC enables the odd radices 7 and 13 (needed only for externally imposed ring lengths);
 // lengths chosen internally are 2-3-5 smooth and use radices 8, 4, 2, 3, 5.
 // R16 enables radix-16 stages (lengths planned with FftLength::init(n, true)); they cost 64 VGPRs of values per
-// butterfly in FP64, so only kernels with the register room (the 1024-thread DFS passes) turn them on.
+// butterfly in FP64, so only the FP32 DFS passes (of every workgroup size) turn them on.
 template <typename T, int NT, int NMAX, bool GENERIC, bool SI, bool SO, bool R16 = false>
 __device__ __forceinline__ void fft_stage_r(c2_t<T>* buf, const FftDesc<T>& d, int R, int ns) {
   if constexpr (R16) {

@@ -1587,7 +1587,7 @@ constexpr long kRowWaves = 4096;
 // more for the denser kernels.  In three processes each over lmax 64 to 4095, measured on zeros and one kernel after the
 // other the tuner took row broadcasts at lmax 1500 spin 2 (0.51 ms, few groups 0.47) in two and more groups at lmax 4095
 // spin 0 (2.73 ms, row broadcasts 2.45) in one; on data, with every kernel run before the first is timed, in none.
-__global__ void k_tuning_alm(double2* __restrict__ alm, long n) {
+static __global__ void k_tuning_alm(double2* __restrict__ alm, long n) {
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
     const unsigned h = (unsigned)i * 2654435761u;
     alm[i] = double2{(h >> 16) * 0x1p-15 - 1.0, (h & 0xffffu) * 0x1p-15 - 1.0};
@@ -1717,7 +1717,7 @@ void legendre_adjoint(const LegendreTables& t, int ncomp, const double2* G, long
   a.st_k = t.st_k.as<double2>();
   a.start = t.start.as<int>();
   a.G = G; a.sm = sm; a.sr = sr; a.alm = alm; a.cnorm = t.cnorm.as<double>();
-  // the lmax that the adjoint is built and checked for
+  // the limits of the range this entry point takes; nothing above them is tested
   NUSHT_REQUIRE(t.lmax <= (t.spin ? 5119 : 10239), kErrUnsupported, "legendre_adjoint: lmax too large");
   StageScope sc(t.n_adj.c_str(), st);
   if (t.spin == 0) launch_adjoint<kScalar>(t, a, st);
